@@ -11,7 +11,10 @@ struct TreeNodeX;
 
 constexpr int kTraceBlock = 128;   // lanes per block of the trace and shadow kernels
 constexpr int kShadeBlock = 128;
+constexpr uint32_t kMaxDepth = 1024;   // largest maxPathDepth
 
+// One block of these counters per bounce of a pass (a path that goes on from
+// bounce b is counted in block b + 1; the ray queues q0 / q1 alternate).
 enum : uint32_t {
     CNT_QUEUE0 = 0, CNT_QUEUE1 = 1, CNT_SHADOW = 2,
     CNT_HIT = 3,                               // hits of shading class 0 (all hits when unsorted)
@@ -116,7 +119,7 @@ struct Frame1 {
     PathBuffers p;
     int* spill;              // traversal-stack spill columns of the trace/shadow grid
     uint32_t spillStride;    // lanes of the trace/shadow grid
-    uint32_t* counters;
+    uint32_t* counters;      // the bounce's block of CNT_COUNT counters
     unsigned long long* stats;
     // path guiding (guided renders only)
     uint32_t guided;          // one-sample MIS with the network at ComplexSurface vertices

@@ -49,7 +49,7 @@ size_t layout_paths(char* base, size_t P, PathBuffers* pb, uint32_t** counters, 
     pb->mq = reinterpret_cast<uint32_t*>(take(P * 4));
     pb->prec = reinterpret_cast<uint32_t*>(take(P * 4));
     pb->sq = reinterpret_cast<uint32_t*>(take(P * 4));
-    *counters = reinterpret_cast<uint32_t*>(take(CNT_COUNT * 4));
+    *counters = reinterpret_cast<uint32_t*>(take((kMaxDepth + 1) * CNT_COUNT * 4));
     *stats = reinterpret_cast<unsigned long long*>(take(STAT_COUNT * 8));
     return off;
 }
@@ -410,7 +410,7 @@ int check_scene(rbh_ctx c, const rbh_launch_params* lp) {
     if (!c->haveColor || !c->haveLuts) return fail(c, RBH_ERR_STATE, "colour tables and LUTs must be uploaded first");
     if (lp->width == 0 || lp->height == 0) return fail(c, RBH_ERR_INVALID, "empty film");
     if ((uint64_t)lp->width * lp->height > (1ull << 28)) return fail(c, RBH_ERR_RANGE, "film above 2^28 pixels");
-    if (lp->maxPathDepth == 0 || lp->maxPathDepth > 1024) return fail(c, RBH_ERR_INVALID, "maxPathDepth must be in [1, 1024]");
+    if (lp->maxPathDepth == 0 || lp->maxPathDepth > kMaxDepth) return fail(c, RBH_ERR_INVALID, "maxPathDepth must be in [1, 1024]");
     if (c->tree.stale || c->tree.nshapes != c->shapes.n)
         return fail(c, RBH_ERR_STATE, "shape lights changed since the light tree was built: rebuild the light tree");
     if (c->geom.maxLight >= (int64_t)c->tree.nlights)
