@@ -35,8 +35,10 @@ struct Hit {
     uint32_t leaf;   // leaf-order triangle record of the hit; 0xFFFFFFFF: miss
 };
 
-__device__ __forceinline__ bool tri_hit(const RayShear& s, V3 o, const TriRecord& tr, float tmax, float& t, float& b1,
-                                        float& b2) {
+// A hit at or before tmax; T and det give its distance as the unrounded
+// quotient t = T / det.
+__device__ __forceinline__ bool tri_candidate(const RayShear& s, V3 o, const TriRecord& tr, float tmax, float& T,
+                                              float& det, float& t, float& b1, float& b2) {
     // No FMA contraction: the 2D edge functions of a shared edge must round
     // identically from both triangles for the test to stay watertight.
 #pragma clang fp contract(off)
@@ -54,9 +56,9 @@ __device__ __forceinline__ bool tri_hit(const RayShear& s, V3 o, const TriRecord
         W = (float)((double)Bx * Ay - (double)By * Ax);
     }
     if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
-    float det = U + V + W;
+    det = U + V + W;
     if (det == 0.0f) return false;
-    float T = U * (s.Sz * Akz) + V * (s.Sz * Bkz) + W * (s.Sz * Ckz);
+    T = U * (s.Sz * Akz) + V * (s.Sz * Bkz) + W * (s.Sz * Ckz);
     if (det < 0.0f) { T = -T; det = -det; V = -V; W = -W; }
     if (T < 0.0f || T > tmax * det) return false;
     const float r = 1.0f / det;
@@ -64,6 +66,11 @@ __device__ __forceinline__ bool tri_hit(const RayShear& s, V3 o, const TriRecord
     b1 = V * r;
     b2 = W * r;
     return true;
+}
+__device__ __forceinline__ bool tri_hit(const RayShear& s, V3 o, const TriRecord& tr, float tmax, float& t, float& b1,
+                                        float& b2) {
+    float T, det;
+    return tri_candidate(s, o, tr, tmax, T, det, t, b1, b2);
 }
 
 // Traversal stack of at most kMaxStack entries (the LBVH builder rejects

@@ -145,8 +145,8 @@ __device__ __forceinline__ void snapshot_radiance(const Frame1& f, uint32_t pid,
 // A path whose ray left the scene: sky emission with the MIS weight of the
 // previous vertex's BxDF sample, then the path ends (pathtrace.cu:1185-1274,
 // the sky branch; 1240-1252 for the lookup and its pdf).
-__device__ __forceinline__ void shade_miss(const Frame1& f, const SceneView& S, uint32_t pid) {
-    const bool first = f.bounce == 0u;
+// first: the path is at its camera ray (its state is fresh, not in memory).
+__device__ __forceinline__ void shade_miss(const Frame1& f, const SceneView& S, uint32_t pid, bool first) {
     float4 nf = first ? init_nf() : f.p.nf[pid];
     uint32_t flags = __float_as_uint(nf.w);
     flags &= ~PF_TRIANGULAR;
@@ -180,6 +180,10 @@ __device__ __forceinline__ void shade_miss(const Frame1& f, const SceneView& S, 
     flags |= PF_FINISHED;
     nf.w = __uint_as_float(flags);
     f.p.nf[pid] = nf;
+}
+
+__device__ __forceinline__ void shade_miss(const Frame1& f, const SceneView& S, uint32_t pid) {
+    shade_miss(f, S, pid, f.bounce == 0u);
 }
 
 // Network input of a hit: scene-normalised position, geometric normal turned
@@ -291,15 +295,16 @@ __device__ __forceinline__ void quat_cols(float4 q, V3& c0, V3& c2) {
 // the path goes on and shadow when it has a shadow ray to test; in guided
 // renders that collect training data, recordSlot with the recorded direction,
 // its BSDF-sampler density and the throughput before the vertex. The outputs
-// must be initialised by the caller (false / zero).
+// must be initialised by the caller (false / zero). first: the path is at its
+// camera ray's hit (its state is fresh, not in memory).
 template <bool GUIDED>
-__device__ __forceinline__ void shade_hit(const Frame1& f, const SceneView& S, uint32_t pid, uint32_t i, bool& alive,
-                                          bool& shadow, bool& recordSlot, V3& recDir, float& recPb, S4& recT) {
+__device__ __forceinline__ void shade_hit(const Frame1& f, const SceneView& S, uint32_t pid, uint32_t i, bool first,
+                                          bool& alive, bool& shadow, bool& recordSlot, V3& recDir, float& recPb,
+                                          S4& recT) {
     const ColorTables ct{S.colors};
     const Luts lut{S.luts};
     const LightTree tree{S.treeNodes, S.treePointers, S.treeMasks, S.envOn != 0};
     const bool treeOn = S.treeNodes != nullptr;
-    const bool first = f.bounce == 0u;
     const float4 od = f.p.od[pid], dr = f.p.dr[pid], nf = first ? init_nf() : f.p.nf[pid], hr = f.p.hit[pid];
     PathIO P;
     P.rd = V3{dr.x, dr.y, dr.z};
@@ -701,6 +706,12 @@ __device__ __forceinline__ void shade_hit(const Frame1& f, const SceneView& S, u
     f.p.dr[pid] = make_float4(P.rd.x, P.rd.y, P.rd.z, P.refr);
     f.p.nf[pid] = make_float4(lastN.x, lastN.y, lastN.z, __uint_as_float(P.flags));
     f.p.depth[pid] = depth;
+}
+
+template <bool GUIDED>
+__device__ __forceinline__ void shade_hit(const Frame1& f, const SceneView& S, uint32_t pid, uint32_t i, bool& alive,
+                                          bool& shadow, bool& recordSlot, V3& recDir, float& recPb, S4& recT) {
+    shade_hit<GUIDED>(f, S, pid, i, f.bounce == 0u, alive, shadow, recordSlot, recDir, recPb, recT);
 }
 
 // Turns the pending records of a finished path into training records. The

@@ -11,6 +11,7 @@ struct TreeNodeX;
 
 constexpr int kTraceBlock = 128;   // lanes per block of the trace and shadow kernels
 constexpr int kShadeBlock = 128;
+constexpr int kPathBlock = 64;
 constexpr uint32_t kMaxDepth = 1024;   // largest maxPathDepth
 
 // One block of these counters per bounce of a pass (a path that goes on from
@@ -115,6 +116,7 @@ struct Frame1 {
     uint32_t bounce;
     uint32_t camOrigin0;          // no scene of the pass uses depth of field: camera rays start at 0
     uint32_t sortHits;            // LaunchShape::sortHits
+    uint32_t tail;                // queues of at most so many paths are run to their end by k_paths (0: none)
     // state
     PathBuffers p;
     int* spill;              // traversal-stack spill columns of the trace/shadow grid

@@ -26,6 +26,7 @@
 #include "../context.hpp"
 #include "../device/mlp_wave.hpp"
 #include "../device/traverse.hpp"
+#include "../device/traverse_quad.hpp"
 #include "../device/wavefront.hpp"
 #include "../integrator.hpp"
 
@@ -239,6 +240,7 @@ __global__ __launch_bounds__(kTraceBlock, WAVES) void k_trace(Frame1 f, uint32_t
     __shared__ uint8_t stagedCls[2 * kTraceBlock];     // per wave: the hits' shading classes
     const TravStack<kStackLds> st = lane_stack(f, stack);
     const uint32_t count = f.counters[qsel ? CNT_QUEUE1 : CNT_QUEUE0];
+    if (f.bounce > 0u && count <= f.tail) return;   // k_paths ran these paths to their end
     const uint32_t* __restrict__ queue = qsel ? f.p.q1 : f.p.q0;
     const bool identity = f.bounce == 0;
     uint32_t nrays = 0;
@@ -459,6 +461,76 @@ __global__ __launch_bounds__(kShadeBlock, WAVES) void k_shade(Frame1 f, uint32_t
     wave_count(f.stats + STAT_VERTICES, nvert);
 }
 
+// ------------------------------------------------------ few paths: one kernel
+// All remaining bounces of the queued paths in one launch, from closest hit
+// to shadow ray, four lanes per path, for queues too short to fill the chip: a
+// bounce of the separate kernels then takes as long as the slowest wave of
+// each of them (about 200 us however few the paths); here a wave only waits
+// for its own 16 paths, and their walks take one box and one triangle per
+// lane (traverse_quad.hpp). The four lanes shade their path redundantly, with
+// the same values, and only the first one counts. State and per-path bodies
+// are those of the separate kernels, so a path's values do not depend on
+// which form ran it. Bound by the latency of a path's chain of bounces: one
+// sample of a 64x64 Cornell box at depth 8 takes 0.42 ms against 1.27 ms in
+// the separate kernels (0.68 ms with one lane per path), 640x360 over 1M
+// triangles with a refit 3.9 against 5.3 ms. bounce: the bounce the queue
+// belongs to (0: every slot starts with its camera ray).
+// kTailPaths: 4096 waves, two resident rounds of the kernel's two waves per
+// SIMD. Measured at 16k / 64k / 128k / 256k paths: 256x256x16 Cornell 3.68 /
+// 3.61 / 3.72 / 4.10 ms, feature scene 333x187x8 2.40 / 2.36 / 2.53 / 2.92 ms,
+// 1080p x 64 spp of 4.1M triangles 114.3 / 114.1 / 116.3 / 122.3 ms.
+constexpr uint32_t kTailPaths = 65536u;
+template <bool BATCH>
+__global__ __launch_bounds__(kPathBlock) void k_paths(Frame1 f, uint32_t bounce, uint32_t depthMax) {
+    __shared__ int stack[kQuadStackLds * kQuadRays];
+    const uint32_t t = (blockIdx.x * kPathBlock + threadIdx.x) >> 2;
+    const TravStack<kQuadStackLds> st{stack + (threadIdx.x >> 2), kQuadRays, f.spill + t, f.spillStride};
+    const uint32_t qsel = bounce & 1u;
+    const uint32_t count = f.counters[qsel ? CNT_QUEUE1 : CNT_QUEUE0];
+    if (count > f.tail) return;   // long enough for the separate kernels
+    const uint32_t* __restrict__ queue = qsel ? f.p.q1 : f.p.q0;
+    uint32_t nclosest = 0, nshadow = 0, nvert = 0;
+    for (uint32_t i = t; i < count; i += gridDim.x * kQuadRays) {
+        const uint32_t pid = bounce == 0u ? i : queue[i];
+        const SceneView& S = scene_of<BATCH>(f, pid);
+        bool alive = true;
+        for (uint32_t b = bounce; alive && b < depthMax; ++b) {
+            V3 o, d;
+            pass_ray<BATCH>(f, S, pid, b == 0u, o, d);
+            float ts = 3.402823466e+38f;
+            uint32_t shape = 0xFFFFFFFFu;
+            if (S.nshapes) shape_closest(S.shapes, S.nshapes, o, d, ts, ts, shape);
+            Hit h = traverse4_quad<false>(S.nodes4, S.tris, S.nnodes4, o, d, ts, st);
+            if (h.leaf == 0xFFFFFFFFu && shape != 0xFFFFFFFFu) h = Hit{ts, 0.0f, 0.0f, shape};
+            ++nclosest;
+            alive = false;
+            if (h.leaf == 0xFFFFFFFFu) {
+                shade_miss(f, S, pid, b == 0u);
+                continue;
+            }
+            f.p.hit[pid] = make_float4(h.t, h.b1, h.b2, __uint_as_float(h.leaf));
+            ++nvert;
+            bool shadow = false, rec = false;
+            V3 recDir{0.0f, 0.0f, 0.0f};
+            float recPb = 0.0f;
+            S4 recT = s4(0.0f);
+            shade_hit<false>(f, S, pid, i, b == 0u, alive, shadow, rec, recDir, recPb, recT);
+            if (shadow) {
+                const float4 so = f.p.sro[pid], sd = f.p.srd[pid];
+                const V3 so3{so.x, so.y, so.z}, sd3{sd.x, sd.y, sd.z};
+                if (!(S.nshapes && shape_any(S.shapes, S.nshapes, so3, sd3, so.w)) &&
+                    traverse4_quad<true>(S.nodes4, S.tris, S.nnodes4, so3, sd3, so.w, st).leaf == 0xFFFFFFFFu)
+                    add_nee(f, pid);
+                ++nshadow;
+            }
+        }
+    }
+    const bool first = (threadIdx.x & 3u) == 0u;
+    wave_count(f.stats + STAT_CLOSEST, first ? nclosest : 0u);
+    wave_count(f.stats + STAT_SHADOW, first ? nshadow : 0u);
+    wave_count(f.stats + STAT_VERTICES, first ? nvert : 0u);
+}
+
 // ----------------------------------------------------------- accumulation
 template <bool BATCH>
 __global__ __launch_bounds__(256) void k_accumulate(Frame1 f) {
@@ -564,10 +636,21 @@ static hipError_t launch_pass_t(rbh_ctx c, Frame1 f, uint32_t depthMax, const La
     uint32_t* const counters = f.counters;
     const uint32_t ncount = (depthMax + 1u) * CNT_COUNT;
     hipLaunchKernelGGL(k_pass_start, dim3((ncount + 255u) / 256u), dim3(256), 0, c->stream, f, ncount);
-    for (uint32_t b = 0; b < depthMax; ++b) {
+    // k_paths: launched before each later bounce of an unguided pass, it leaves
+    // at once unless the queue has become short; a pass short from the start
+    // is that one launch. Per-kernel timing keeps the kernels apart.
+    f.tail = f.guided || kt ? 0u : kTailPaths;
+    // (no more lanes than the trace grid's spill columns)
+    const dim3 pathGrid(std::min<uint32_t>((std::min(std::max(f.tail, 1u), f.NP) + kQuadRays - 1) / kQuadRays,
+                                           (uint32_t)ls.traceGrid * kTraceBlock / kQuadRays));
+    const bool allPaths = f.NP <= f.tail;
+    if (allPaths) hipLaunchKernelGGL((k_paths<BATCH>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
+    for (uint32_t b = 0; b < depthMax && !allPaths; ++b) {
         const uint32_t qsel = b & 1u;
         f.bounce = b;
         f.counters = counters + b * CNT_COUNT;
+        if (f.tail && b > 0)
+            hipLaunchKernelGGL((k_paths<BATCH>), pathGrid, dim3(kPathBlock), 0, c->stream, f, b, depthMax);
         RBH_TIMED(KernelTimer::TRACE, launch_trace<BATCH>(c, f, qsel, ls));
         RBH_TIMED(KernelTimer::SHADE,
                   hipLaunchKernelGGL(k_miss<BATCH>, dim3(ls.shadeGrid), dim3(256), 0, c->stream, f));

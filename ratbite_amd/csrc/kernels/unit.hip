@@ -19,6 +19,7 @@
 #include "../device/lighttree.hpp"
 #include "../device/qrng.hpp"
 #include "../device/traverse.hpp"
+#include "../device/traverse_quad.hpp"
 #include "radix.hpp"
 
 namespace rbh {
@@ -88,6 +89,25 @@ __global__ __launch_bounds__(128) void k_trace_test(const BvhNode* nodes, const 
     const Hit h = tree == 1 ? traverse<ANY>(nodes, tris, nnodes, ro, rd, r[7], st)
                 : tree == 2 ? traverse4<ANY>(nodes4q, tris, nnodes4, ro, rd, r[7], st)
                             : traverse4<ANY>(nodes4, tris, nnodes4, ro, rd, r[7], st);
+    float* o = hits + 4 * (size_t)i;
+    o[0] = h.leaf == 0xFFFFFFFFu ? -1.0f : h.t;
+    o[1] = __uint_as_float(h.leaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : tris[h.leaf].prim);
+    o[2] = h.b1;
+    o[3] = h.b2;
+}
+
+// the four-lanes-per-ray walk, 32 rays per block
+template <bool ANY, int LDS_DEPTH>
+__global__ __launch_bounds__(128) void k_trace_quad_test(const Bvh4Node* nodes4, const TriRecord* tris, uint32_t nn4,
+                                                         const float* rays, float* hits, uint32_t n, int* spill,
+                                                         uint32_t spillStride) {
+    __shared__ int stack[LDS_DEPTH * 32];
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 2;
+    if (i >= n) return;
+    const TravStack<LDS_DEPTH> st{stack + (threadIdx.x >> 2), 32, spill + i, spillStride};
+    const float* r = rays + 8 * (size_t)i;
+    const Hit h = traverse4_quad<ANY>(nodes4, tris, nn4, V3{r[0], r[1], r[2]}, V3{r[4], r[5], r[6]}, r[7], st);
+    if (threadIdx.x & 3u) return;
     float* o = hits + 4 * (size_t)i;
     o[0] = h.leaf == 0xFFFFFFFFu ? -1.0f : h.t;
     o[1] = __uint_as_float(h.leaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : tris[h.leaf].prim);
@@ -292,6 +312,18 @@ int rbh_test_trace(rbh_ctx c, const float* rays, float* hits, uint32_t n, int mo
     const TriRecord* tris = c->accel.tris.as<TriRecord>();
     const uint32_t nn = c->accel.nnodes, nn4 = c->accel.nnodes4;
     const bool any = (mode & 1) != 0, tiny = (mode & 2) != 0;
+    if (mode & 16) {
+        // four lanes per ray
+        const dim3 gq = grid(n, 32);
+        const uint32_t cols = gq.x * 32u;
+        int* sq = (int*)s.out((size_t)cols * kMaxStack4 * 4);
+        STAGE_CHECK(sq);
+        auto k = any ? (tiny ? k_trace_quad_test<true, 2> : k_trace_quad_test<true, kQuadStackLds>)
+                     : (tiny ? k_trace_quad_test<false, 2> : k_trace_quad_test<false, kQuadStackLds>);
+        hipLaunchKernelGGL(k, gq, dim3(128), 0, 0, nodes4, tris, nn4, (const float*)dr, (float*)dh, n, sq, cols);
+        FINISH(hits, dh, (size_t)n * 16);
+        return RBH_OK;
+    }
     const int binary = (mode & 4) ? 1 : ((mode & 8) ? 2 : 0);
     // mode bit 1: a 2-entry LDS stack, so the spill columns carry the rest;
     // bit 2: the binary tree instead of the four-wide one; bit 3: the
