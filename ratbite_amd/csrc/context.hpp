@@ -78,8 +78,9 @@ struct Accel {
     uint32_t nnodes = 0, depth = 0;
     DevBuf nodes;     // BvhNode (binary LBVH)
     DevBuf nodes4;    // Bvh4Node (the binary tree collapsed four-wide; traversed)
-    DevBuf nodes4q;   // the four-wide nodes quantised to 64 bytes (Bvh4QNode)
-    uint32_t nnodes4 = 0;
+    DevBuf nodes4q;   // the four-wide nodes quantised to 64 bytes (Bvh4QNode), made when a render traverses them
+    bool quantised = false;
+    uint32_t nnodes4 = 0;    // indices of four-wide nodes are below (with gaps)
     DevBuf tris;      // TriRecord in leaf order
     DevBuf scratch;   // build scratch
     size_t keysOffset = 0;   // byte offset of the sorted 64-bit keys in scratch (kept after the build)

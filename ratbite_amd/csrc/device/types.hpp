@@ -21,21 +21,21 @@ constexpr size_t kLutTotal = kLutSheen + 32 * 32 * 4;
 
 // Binary BVH node, 64 bytes: both children's boxes in one node so a
 // traversal step is one 64-byte fetch (two dwordx4 pairs).
-// child >= 0: inner node index; child < 0: ~(first triangle) with the
-// triangle count in the low bits of cnt.
+// child >= 0: inner node index; child < 0: ~triangle.
 struct alignas(16) BvhNode {
     float lminx, lmaxx, lminy, lmaxy;   // left child box (x, y)
     float rminx, rmaxx, rminy, rmaxy;   // right child box (x, y)
     float lminz, lmaxz, rminz, rmaxz;   // z extents
     int32_t left, right;                // child references
-    uint32_t lcnt, rcnt;                // triangle counts of leaf children (0 = inner)
+    uint32_t lcnt, rcnt;                // triangles below each child
 };
 static_assert(sizeof(BvhNode) == 64, "BvhNode is 64 bytes");
 
 // Four-wide BVH node, 128 bytes (one 128-byte cache line): the boxes of up to
 // four children as structure-of-arrays rows, then the child references
 // (>= 0 inner node, < 0 ~leaf index into the triangle records, kBvh4Empty
-// for an unused slot, whose box is empty: lo = +inf, hi = -inf).
+// for an unused slot, whose box is empty: lo = +inf, hi = -inf). The inner
+// children of a node have consecutive indices, in slot order.
 constexpr int32_t kBvh4Empty = (int32_t)0x80000000;
 struct alignas(16) Bvh4Node {
     float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];

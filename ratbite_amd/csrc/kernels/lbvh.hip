@@ -9,15 +9,19 @@
 //   3. stable LSD radix sort of the keys (radix.hpp: ballot-ranked 8-bit digits)
 //   4. Karras (HPG 2012) hierarchy: internal node i covers a key range and
 //      splits at the highest differing bit
-//   5. refit level by level from the deepest internal nodes up (one launch
-//      per depth, so kernel boundaries order the box writes; no cross-XCD
-//      fences or arrival counters); node depths by pointer jumping, the
-//      depth order by a radix sort of (depth, node) pairs
-//   6. emission of 64-byte two-child nodes (both child boxes in the parent)
-//      and of triangles in leaf order
-//   7. collapse into 128-byte four-wide nodes, top down one level per launch:
-//      a four-wide node takes its binary node's children and keeps opening
-//      the inner child with the largest box surface until it has four
+//   5. boxes bottom up: a workgroup takes 2048 consecutive leaves, writes their
+//      triangle records and climbs the hierarchy in LDS (of a node's two
+//      children the second to arrive merges them) as far as the nodes' leaf
+//      ranges stay within the workgroup's; one workgroup then climbs the few
+//      nodes above (no cross-XCD fences: only kernel boundaries order the
+//      two). A node is emitted where its children meet, as the 64-byte
+//      two-child node with both child boxes
+//   6. collapse into 128-byte four-wide nodes, top down: a four-wide node
+//      takes its binary node's children and keeps opening the inner child
+//      with the largest box surface until it has four. The same workgroup
+//      runs the upper levels, then one wave per subtree finishes. The inner
+//      children of a four-wide node have consecutive indices in slot order,
+//      from a range of indices that belongs to the node alone
 // Every root-to-leaf path strictly lengthens the common key prefix, so the
 // depth is at most 64 and a 64-entry traversal stack never overflows.
 #include "../context.hpp"
@@ -40,9 +44,11 @@ __device__ __forceinline__ float ord2f(uint32_t u) {
 __global__ void k_bounds_init(uint32_t* __restrict__ b) {
     if (threadIdx.x < 3) b[threadIdx.x] = 0xFFFFFFFFu;           // min (ordered)
     else if (threadIdx.x < 6) b[threadIdx.x] = 0u;               // max (ordered)
-    else if (threadIdx.x == 6) b[6] = 0u;                         // depth
 }
 
+// One set of six atomics per workgroup, all on one line (2048 workgroups
+// waited 140 us for them, 512 do not)
+constexpr int kBoundsBlocks = 512;
 __global__ __launch_bounds__(kBuildBlock) void k_centroid_bounds(const float* __restrict__ v, const uint32_t* __restrict__ idx,
                                                                  uint32_t n, uint32_t* __restrict__ b) {
     __shared__ float smin[3][kBuildBlock], smax[3][kBuildBlock];
@@ -115,11 +121,15 @@ __device__ __forceinline__ int common_prefix(const unsigned long long* __restric
     return __clzll(k[i] ^ k[j]);
 }
 
+// Parent link of a binary subtree: the parent's index and the side of the
+// child (1: right); kNoParent for the root.
+constexpr uint32_t kNoParent = 0xFFFFFFFFu;
+
 // Karras 2012, Figure 4. Internal nodes 0..n-2; child ids >= 0 internal,
-// < 0 leaf ~sortedIndex. parent[] holds internal parents of internal nodes
+// < 0 leaf ~sortedIndex. parent[] holds the parent links of internal nodes
 // (slot i) and of leaves (slot n-1+j).
 __global__ __launch_bounds__(kBuildBlock) void k_karras(const unsigned long long* __restrict__ k, int n,
-                                                        int2* __restrict__ child, int* __restrict__ parent) {
+                                                        uint32_t* __restrict__ parent) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
     const int d = (common_prefix(k, n, i, i + 1) - common_prefix(k, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -139,132 +149,166 @@ __global__ __launch_bounds__(kBuildBlock) void k_karras(const unsigned long long
     } while (t > 1);
     const int split = i + s * d + min(d, 0);
     const int first = min(i, j), last = max(i, j);
-    const int left = (first == split) ? ~split : split;
-    const int right = (last == split + 1) ? ~(split + 1) : split + 1;
-    child[i] = make_int2(left, right);
-    if (left >= 0) parent[left] = i; else parent[n - 1 + split] = i;
-    if (right >= 0) parent[right] = i; else parent[n - 1 + split + 1] = i;
-    if (i == 0) parent[0] = -1;
+    parent[first == split ? n - 1 + split : split] = (uint32_t)i << 1;
+    parent[last == split + 1 ? n - 1 + split + 1 : split + 1] = ((uint32_t)i << 1) | 1u;
+    if (i == 0) parent[0] = kNoParent;
 }
 
 struct Box { float lo[3], hi[3]; };
 
-// Triangle records in leaf (Morton) order and their boxes.
-__global__ __launch_bounds__(kBuildBlock) void k_leaves(const float* __restrict__ v, const uint32_t* __restrict__ idx,
-                                                        const uint32_t* __restrict__ triMaterial,
-                                                        const uint32_t* __restrict__ triLight,
-                                                        const Material* __restrict__ mats, uint32_t nmats,
-                                                        const unsigned long long* __restrict__ keys, int n, int idxBits,
-                                                        float* __restrict__ lbox, TriRecord* __restrict__ tris) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const uint32_t tri = (uint32_t)(keys[j] & ((1ull << idxBits) - 1ull));
-    const uint32_t a = idx[3 * tri], b = idx[3 * tri + 1], c = idx[3 * tri + 2];
-    TriRecord r;
-    r.v0x = v[3 * a]; r.v0y = v[3 * a + 1]; r.v0z = v[3 * a + 2]; r.prim = tri;
-    r.v1x = v[3 * b]; r.v1y = v[3 * b + 1]; r.v1z = v[3 * b + 2]; r.material = triMaterial[tri];
-    r.v2x = v[3 * c]; r.v2y = v[3 * c + 1]; r.v2z = v[3 * c + 2]; r.light = triLight[tri];
-    r.i0 = a; r.i1 = b; r.i2 = c;
-    r.shadeClass = r.material < nmats ? shade_class(mats[r.material]) : (uint32_t)SC_SURFACE;
-    tris[j] = r;
-    float* lb = lbox + 6 * (size_t)j;
-    lb[0] = fminf(fminf(r.v0x, r.v1x), r.v2x); lb[3] = fmaxf(fmaxf(r.v0x, r.v1x), r.v2x);
-    lb[1] = fminf(fminf(r.v0y, r.v1y), r.v2y); lb[4] = fmaxf(fmaxf(r.v0y, r.v1y), r.v2y);
-    lb[2] = fminf(fminf(r.v0z, r.v1z), r.v2z); lb[5] = fmaxf(fmaxf(r.v0z, r.v1z), r.v2z);
+__device__ __forceinline__ Box merge(const Box& a, const Box& b) {
+    Box r;
+    for (int k = 0; k < 3; ++k) {
+        r.lo[k] = fminf(a.lo[k], b.lo[k]);
+        r.hi[k] = fmaxf(a.hi[k], b.hi[k]);
+    }
+    return r;
 }
 
-constexpr int kLevels = 65;   // internal-node depths 0..63 (64 collects anything deeper)
+// Box and reference of one side of a two-child node.
+__device__ __forceinline__ Box node_half(const BvhNode& nd, uint32_t side) {
+    return side ? Box{{nd.rminx, nd.rminy, nd.rminz}, {nd.rmaxx, nd.rmaxy, nd.rmaxz}}
+                : Box{{nd.lminx, nd.lminy, nd.lminz}, {nd.lmaxx, nd.lmaxy, nd.lmaxz}};
+}
+__device__ __forceinline__ void put_half(BvhNode* __restrict__ nd, uint32_t side, const Box& b, int ref, uint32_t tris) {
+    if (side) {
+        nd->rminx = b.lo[0]; nd->rmaxx = b.hi[0]; nd->rminy = b.lo[1]; nd->rmaxy = b.hi[1];
+        nd->rminz = b.lo[2]; nd->rmaxz = b.hi[2];
+        nd->right = ref;
+        nd->rcnt = tris;
+    } else {
+        nd->lminx = b.lo[0]; nd->lmaxx = b.hi[0]; nd->lminy = b.lo[1]; nd->lmaxy = b.hi[1];
+        nd->lminz = b.lo[2]; nd->lmaxz = b.hi[2];
+        nd->left = ref;
+        nd->lcnt = tris;
+    }
+}
 
-// Depth of every internal node (ancestors up to the root) and a histogram.
-// Depth of every internal node by pointer jumping over the parent links:
-// (ancestor, distance) pairs, each round adds the ancestor's distance and
-// jumps to the ancestor's ancestor, so ceil(log2(64)) + 1 = 7 rounds reach the
-// root from depth 64 (deeper trees are rejected after the build).
-constexpr int kJumpRounds = 7;
-__global__ __launch_bounds__(kBuildBlock) void k_jump_init(int nInt, const int* __restrict__ parent,
-                                                           int2* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nInt) return;
-    const int p = parent[i];
-    out[i] = make_int2(p, p >= 0 ? 1 : 0);
+// A finished subtree that a workgroup hands on: its parent is not one of the
+// nodes with the workgroup's own indices. Lists of them are kept per group of
+// kGroupTiles leaf tiles. A workgroup hands on at most one subtree per level
+// on either side of its leaves (the parents' ranges are nested), or the root.
+struct Pending {
+    Box box;
+    int ref;            // node, or ~leaf
+    uint32_t parent;    // parent link
+    uint32_t height;    // inner nodes on its longest path down
+    uint32_t tris;
+};
+// counters of the build's last stages
+constexpr int kCollapseRounds = 4;
+enum : int { BC_DEPTH = 0, BC_TOP = 1, BC_QUEUE = 2, BC_COUNT = BC_QUEUE + kCollapseRounds + 1 };
+constexpr int kLeafTile = 2048;
+constexpr int kGroupTiles = 32;
+constexpr int kGroupLeaves = kGroupTiles * kLeafTile;
+constexpr int kHandedOn = 130;   // most subtrees one workgroup hands on (trees of at most 64 levels)
+
+// cnt: the counters above, then the length of every group's list
+__global__ __launch_bounds__(kBuildBlock) void k_build_counters(uint32_t* __restrict__ cnt, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) cnt[i] = 0u;
 }
-__global__ __launch_bounds__(kBuildBlock) void k_jump(int nInt, const int2* __restrict__ in, int2* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nInt) return;
-    const int2 a = in[i];
-    if (a.x < 0) {
-        out[i] = a;
-        return;
+
+// Triangle records in leaf (Morton) order and the boxes of the hierarchy as
+// far as they lie within the workgroup's leaves [first, first + kLeafTile).
+// Every thread starts at its leaves and climbs: at a node the first child to
+// arrive leaves its box in LDS and stops, the second merges the two, emits
+// the node and goes on. An internal node's index is an end of its leaf
+// range, so the nodes a workgroup can finish are the ones with its leaves'
+// indices; a subtree whose parent lies elsewhere is handed on, and of the
+// workgroup's own nodes that stay incomplete the arrived half is stored for
+// the climb above. Bound by the records' and nodes' 64-byte writes and
+// the vertex gathers.
+constexpr int kLeafBlock = 1024;
+constexpr uint32_t kArrivedLeft = 1u, kArrivedRight = 0x100u;
+__global__ __launch_bounds__(kLeafBlock) void k_leaves(const float* __restrict__ v, const uint32_t* __restrict__ idx,
+                                                       const uint32_t* __restrict__ triMaterial,
+                                                       const uint32_t* __restrict__ triLight,
+                                                       const Material* __restrict__ mats, uint32_t nmats,
+                                                       const unsigned long long* __restrict__ keys, int n, int idxBits,
+                                                       const uint32_t* __restrict__ parent, TriRecord* __restrict__ tris,
+                                                       BvhNode* __restrict__ nodes, uint32_t* __restrict__ arrived,
+                                                       uint32_t* __restrict__ height, Pending* __restrict__ pending,
+                                                       uint32_t* __restrict__ cnt) {
+    __shared__ float sbox[2][6][kLeafTile];
+    __shared__ int sref[2][kLeafTile];
+    __shared__ uint32_t smeta[2][kLeafTile];   // height << 16 | triangles (at most a tile's)
+    __shared__ uint32_t sarrived[kLeafTile], sparent[kLeafTile];
+    const int first = blockIdx.x * kLeafTile;
+    const uint32_t group = blockIdx.x / kGroupTiles;
+    const int own = min(kLeafTile, n - 1 - first);   // internal nodes with the tile's indices
+    for (int k = threadIdx.x; k < kLeafTile; k += kLeafBlock) {
+        sarrived[k] = 0u;
+        sparent[k] = k < own ? parent[first + k] : kNoParent;
     }
-    const int2 b = in[a.x];
-    out[i] = make_int2(b.x, a.y + b.y);
-}
-// sort keys: the depth (capped at kLevels - 1) and the node index
-__global__ __launch_bounds__(kBuildBlock) void k_depth_keys(int nInt, const int2* __restrict__ jumped,
-                                                            unsigned int* __restrict__ key, int* __restrict__ id) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nInt) return;
-    key[i] = (unsigned int)min(jumped[i].y, kLevels - 1);
-    id[i] = i;
-}
-// start[d] = first position of depth d in the depth-sorted order (d <= kLevels)
-__global__ void k_level_bounds(const unsigned int* __restrict__ sortedKey, int nInt, int* __restrict__ start) {
-    const int d = threadIdx.x;
-    if (d > kLevels) return;
-    int lo = 0, hi = nInt;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if ((int)sortedKey[mid] < d) lo = mid + 1;
-        else hi = mid;
-    }
-    start[d] = lo;
-}
-__global__ __launch_bounds__(kBuildBlock) void k_refit_level(int level, const int* __restrict__ start,
-                                                             const int* __restrict__ order, const int2* __restrict__ child,
-                                                             float* __restrict__ ibox, const float* __restrict__ lbox) {
-    const int b = start[level], e = start[level + 1];
-    for (int t = b + blockIdx.x * blockDim.x + threadIdx.x; t < e; t += gridDim.x * blockDim.x) {
-        const int p = order[t];
-        const int2 ch = child[p];
-        const float* A = ch.x >= 0 ? ibox + 6 * (size_t)ch.x : lbox + 6 * (size_t)(~ch.x);
-        const float* B = ch.y >= 0 ? ibox + 6 * (size_t)ch.y : lbox + 6 * (size_t)(~ch.y);
-        float* o = ibox + 6 * (size_t)p;
-        for (int k = 0; k < 3; ++k) {
-            o[k] = fminf(A[k], B[k]);
-            o[3 + k] = fmaxf(A[3 + k], B[3 + k]);
+    __syncthreads();
+    for (int q = threadIdx.x; q < kLeafTile && first + q < n; q += kLeafBlock) {
+        const int j = first + q;
+        const uint32_t tri = (uint32_t)(keys[j] & ((1ull << idxBits) - 1ull));
+        const uint32_t a = idx[3 * (size_t)tri], b = idx[3 * (size_t)tri + 1], c = idx[3 * (size_t)tri + 2];
+        TriRecord r;
+        r.v0x = v[3 * a]; r.v0y = v[3 * a + 1]; r.v0z = v[3 * a + 2]; r.prim = tri;
+        r.v1x = v[3 * b]; r.v1y = v[3 * b + 1]; r.v1z = v[3 * b + 2]; r.material = triMaterial[tri];
+        r.v2x = v[3 * c]; r.v2y = v[3 * c + 1]; r.v2z = v[3 * c + 2]; r.light = triLight[tri];
+        r.i0 = a; r.i1 = b; r.i2 = c;
+        r.shadeClass = r.material < nmats ? shade_class(mats[r.material]) : (uint32_t)SC_SURFACE;
+        tris[j] = r;
+        if (n == 1) break;
+        Pending t;
+        t.box = Box{{fminf(fminf(r.v0x, r.v1x), r.v2x), fminf(fminf(r.v0y, r.v1y), r.v2y), fminf(fminf(r.v0z, r.v1z), r.v2z)},
+                    {fmaxf(fmaxf(r.v0x, r.v1x), r.v2x), fmaxf(fmaxf(r.v0y, r.v1y), r.v2y), fmaxf(fmaxf(r.v0z, r.v1z), r.v2z)}};
+        t.ref = ~j;
+        t.parent = parent[n - 1 + j];
+        t.height = 0u;
+        t.tris = 1u;
+        while (true) {
+            const int p = (int)(t.parent >> 1), k = p - first;
+            const uint32_t side = t.parent & 1u, other = side ^ 1u;
+            if (t.parent == kNoParent || k < 0 || k >= own) {
+                pending[(size_t)group * kGroupTiles * kHandedOn + atomicAdd(cnt + BC_COUNT + group, 1u)] = t;
+                break;
+            }
+            for (int e = 0; e < 3; ++e) {
+                sbox[side][e][k] = t.box.lo[e];
+                sbox[side][3 + e][k] = t.box.hi[e];
+            }
+            sref[side][k] = t.ref;
+            smeta[side][k] = t.height << 16 | t.tris;
+            const uint32_t old = __hip_atomic_fetch_add(&sarrived[k], side ? kArrivedRight : kArrivedLeft, __ATOMIC_ACQ_REL,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (old == 0u) break;
+            const Box ob{{sbox[other][0][k], sbox[other][1][k], sbox[other][2][k]},
+                         {sbox[other][3][k], sbox[other][4][k], sbox[other][5][k]}};
+            const int oref = sref[other][k];
+            const uint32_t om = smeta[other][k], otris = om & 0xFFFFu;
+            const Box lb = side ? ob : t.box, rb = side ? t.box : ob;
+            BvhNode nd;
+            put_half(&nd, 0u, lb, side ? oref : t.ref, side ? otris : t.tris);
+            put_half(&nd, 1u, rb, side ? t.ref : oref, side ? t.tris : otris);
+            nodes[p] = nd;
+            t.box = merge(lb, rb);
+            t.ref = p;
+            t.height = max(t.height, om >> 16) + 1u;
+            t.tris += otris;
+            t.parent = sparent[k];
         }
     }
+    __syncthreads();
+    for (int k = threadIdx.x; k < own; k += kLeafBlock) {
+        const uint32_t got = sarrived[k];
+        if (got == (kArrivedLeft | kArrivedRight)) continue;
+        arrived[first + k] = got ? 1u : 0u;
+        if (!got) continue;
+        const uint32_t side = got == kArrivedRight ? 1u : 0u;
+        put_half(nodes + first + k, side,
+                 Box{{sbox[side][0][k], sbox[side][1][k], sbox[side][2][k]},
+                     {sbox[side][3][k], sbox[side][4][k], sbox[side][5][k]}}, sref[side][k], smeta[side][k] & 0xFFFFu);
+        height[2 * (size_t)(first + k) + side] = smeta[side][k] >> 16;
+    }
 }
 
-// Depth of every leaf (number of internal ancestors); the maximum bounds the
-// traversal stack.
-__global__ __launch_bounds__(kBuildBlock) void k_depth(int n, const int* __restrict__ parent, uint32_t* __restrict__ depthOut) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    uint32_t d = 0;
-    for (int p = n > 1 ? parent[n - 1 + j] : -1; p >= 0 && d < 1000; p = parent[p]) ++d;
-    atomicMax(depthOut, d);
-}
-
-__global__ __launch_bounds__(kBuildBlock) void k_emit(int n, const int2* __restrict__ child, const float* __restrict__ ibox,
-                                                      const float* __restrict__ lbox, BvhNode* __restrict__ nodes) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int2 ch = child[i];
-    const float* A = ch.x >= 0 ? ibox + 6 * (size_t)ch.x : lbox + 6 * (size_t)(~ch.x);
-    const float* B = ch.y >= 0 ? ibox + 6 * (size_t)ch.y : lbox + 6 * (size_t)(~ch.y);
-    BvhNode nd;
-    nd.lminx = A[0]; nd.lmaxx = A[3]; nd.lminy = A[1]; nd.lmaxy = A[4];
-    nd.rminx = B[0]; nd.rmaxx = B[3]; nd.rminy = B[1]; nd.rmaxy = B[4];
-    nd.lminz = A[2]; nd.lmaxz = A[5]; nd.rminz = B[2]; nd.rmaxz = B[5];
-    nd.left = ch.x; nd.right = ch.y;
-    nd.lcnt = ch.x < 0 ? 1u : 0u;
-    nd.rcnt = ch.y < 0 ? 1u : 0u;
-    nodes[i] = nd;
-}
-
-__device__ __forceinline__ float half_area(const float* b) {
-    const float x = b[3] - b[0], y = b[4] - b[1], z = b[5] - b[2];
+__device__ __forceinline__ float half_area(const Box& b) {
+    const float x = b.hi[0] - b.lo[0], y = b.hi[1] - b.lo[1], z = b.hi[2] - b.lo[2];
     return x * y + y * z + z * x;
 }
 
@@ -286,7 +330,7 @@ __device__ __forceinline__ void qnode_bounds(float lo, float s, float clo, float
     while (qhi < 255u && qnode_decode(lo, qhi, s) < chi) ++qhi;
 }
 
-// Quantised copy of a four-wide node (empty slots get zero bytes; their
+// Quantised form of a four-wide node (empty slots get zero bytes; their
 // child reference masks them in traversal).
 __device__ __forceinline__ Bvh4QNode quantise_node(const Bvh4Node& nd) {
     float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -316,73 +360,251 @@ __device__ __forceinline__ Bvh4QNode quantise_node(const Bvh4Node& nd) {
     return q;
 }
 
-// One collapse level: in[] holds (binary node, four-wide index) pairs; each
-// produces its four-wide node and appends its inner children to out[].
-__global__ __launch_bounds__(kBuildBlock) void k_collapse(const int2* __restrict__ child, const float* __restrict__ ibox,
-                                                          const float* __restrict__ lbox, const int2* __restrict__ in,
-                                                          const unsigned int* __restrict__ inCount, int2* __restrict__ out,
-                                                          unsigned int* __restrict__ outCount,
-                                                          unsigned int* __restrict__ nodeCount, Bvh4Node* __restrict__ nodes4,
-                                                          Bvh4QNode* __restrict__ nodes4q) {
-    const unsigned int cnt = *inCount;
-    for (unsigned int t = blockIdx.x * blockDim.x + threadIdx.x; t < cnt; t += gridDim.x * blockDim.x) {
-        const int2 w = in[t];
-        int slot[4];
-        int ns = 2;
-        slot[0] = child[w.x].x;
-        slot[1] = child[w.x].y;
-        while (ns < 4) {
-            int best = -1;
-            float area = -1.0f;
-            for (int k = 0; k < ns; ++k)
-                if (slot[k] >= 0) {
-                    const float a = half_area(ibox + 6 * (size_t)slot[k]);
-                    if (a > area) { area = a; best = k; }
-                }
-            if (best < 0) break;
-            const int2 ch = child[slot[best]];
-            slot[best] = ch.x;
-            slot[ns++] = ch.y;
-        }
-        Bvh4Node nd;
-        for (int k = 0; k < 4; ++k) {
-            if (k >= ns) {
-                nd.lox[k] = nd.loy[k] = nd.loz[k] = INFINITY;
-                nd.hix[k] = nd.hiy[k] = nd.hiz[k] = -INFINITY;
-                nd.child[k] = kBvh4Empty;
-                continue;
+// The most four-wide nodes a subtree of n >= 1 triangles collapses into: a
+// node has four children unless all of them are triangles, so with the bound
+// for its children 1 + sum (2 n_i - 1) / 3 = (2 n - 1) / 3.
+__host__ __device__ __forceinline__ uint32_t max_nodes4(uint32_t n) { return (uint32_t)((2ull * n - 1ull) / 3ull); }
+
+// A four-wide node to write: its index, the binary node it starts at and the
+// first of the max_nodes4(triangles) - 1 indices that are its subtree's. With
+// indices that no other subtree can take, nodes need no shared counter (one
+// atomic per wave step on it made the step 17 us) and a subtree's nodes lie
+// together.
+struct Open {
+    uint32_t id;
+    int node;
+    uint32_t room;
+};
+
+// Writes the four-wide node of t: the two children of its binary node, then
+// again and again the inner child with the largest box surface replaced by
+// its own two, until there are four. Its inner children go to t.room,
+// t.room + 1, ... in slot order, their subtrees' indices follow. Returns the
+// number of inner children, next[0..] the nodes to write for them.
+__device__ __forceinline__ uint32_t collapse_node(const Open& t, const BvhNode* nodes, Bvh4Node* __restrict__ nodes4,
+                                                  Open (&next)[4]) {
+    Box box[4];
+    int ref[4];
+    uint32_t tris[4];
+    {
+        const BvhNode nd = nodes[t.node];
+        box[0] = node_half(nd, 0u);
+        box[1] = node_half(nd, 1u);
+        ref[0] = nd.left;
+        ref[1] = nd.right;
+        tris[0] = nd.lcnt;
+        tris[1] = nd.rcnt;
+    }
+#pragma unroll
+    for (int k = 2; k < 4; ++k) {
+        box[k] = Box{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+        ref[k] = kBvh4Empty;
+        tris[k] = 0u;
+    }
+#pragma unroll
+    for (int ns = 2; ns < 4; ++ns) {
+        int best = -1, open = 0;
+        float area = -1.0f;
+#pragma unroll
+        for (int k = 0; k < ns; ++k)
+            if (ref[k] >= 0) {
+                const float a = half_area(box[k]);
+                if (a > area) { area = a; best = k; open = ref[k]; }
             }
-            const int c = slot[k];
-            const float* b = c >= 0 ? ibox + 6 * (size_t)c : lbox + 6 * (size_t)(~c);
-            nd.lox[k] = b[0]; nd.loy[k] = b[1]; nd.loz[k] = b[2];
-            nd.hix[k] = b[3]; nd.hiy[k] = b[4]; nd.hiz[k] = b[5];
-            if (c >= 0) {
-                const int id = (int)atomicAdd(nodeCount, 1u);
-                nd.child[k] = id;
-                out[atomicAdd(outCount, 1u)] = make_int2(c, id);
-            } else {
-                nd.child[k] = c;
+        if (best < 0) break;
+        const BvhNode nd = nodes[open];
+#pragma unroll
+        for (int k = 0; k < ns; ++k)
+            if (k == best) {
+                box[k] = node_half(nd, 0u);
+                ref[k] = nd.left;
+                tris[k] = nd.lcnt;
             }
+        box[ns] = node_half(nd, 1u);
+        ref[ns] = nd.right;
+        tris[ns] = nd.rcnt;
+    }
+    uint32_t inner = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) inner += ref[k] >= 0 ? 1u : 0u;
+    Bvh4Node out;
+    uint32_t id = t.room, room = t.room + inner, q = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        out.lox[k] = box[k].lo[0]; out.loy[k] = box[k].lo[1]; out.loz[k] = box[k].lo[2];
+        out.hix[k] = box[k].hi[0]; out.hiy[k] = box[k].hi[1]; out.hiz[k] = box[k].hi[2];
+        out.child[k] = ref[k];
+        if (ref[k] >= 0) {
+            const Open o{id, ref[k], room};
+            out.child[k] = (int)id++;
+            room += max_nodes4(tris[k]) - 1u;
+#pragma unroll
+            for (uint32_t e = 0; e <= (uint32_t)k; ++e)
+                if (e == q) next[e] = o;
+            ++q;
         }
-        nd.pad[0] = nd.pad[1] = nd.pad[2] = nd.pad[3] = 0;
-        nodes4[w.y] = nd;
-        nodes4q[w.y] = quantise_node(nd);
+    }
+    out.pad[0] = out.pad[1] = out.pad[2] = out.pad[3] = 0;
+    nodes4[t.id] = out;
+    return inner;
+}
+
+// Sum of v over the lanes below (v <= 4) and over the wave.
+__device__ __forceinline__ uint32_t wave_prefix4(uint32_t v, uint32_t& sum) {
+    const unsigned long long b0 = __ballot(v & 1u), b1 = __ballot(v & 2u), b2 = __ballot(v & 4u);
+    const unsigned long long lt = (1ull << __lane_id()) - 1ull;
+    sum = (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2));
+    return (uint32_t)(__popcll(b0 & lt) + 2 * __popcll(b1 & lt) + 4 * __popcll(b2 & lt));
+}
+
+// One thread's climb from a handed-on subtree over the internal nodes
+// [first, last), whose halves, arrival counts and heights lie in global
+// memory, which one workgroup sees in order. Returns true with t the subtree
+// whose parent lies outside (or the root), false when the other child of a
+// node is still to come.
+__device__ __forceinline__ bool climb(Pending& t, uint32_t first, uint32_t last, const uint32_t* __restrict__ parent,
+                                      BvhNode* nodes, uint32_t* arrived, uint32_t* height) {
+    while (true) {
+        const uint32_t p = t.parent >> 1, side = t.parent & 1u;
+        if (t.parent == kNoParent || p < first || p >= last) return true;
+        const uint32_t up = parent[p];
+        put_half(nodes + p, side, t.box, t.ref, t.tris);
+        height[2 * (size_t)p + side] = t.height;
+        if (__hip_atomic_fetch_add(arrived + p, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u) return false;
+        const BvhNode nd = nodes[p];
+        t.box = merge(node_half(nd, 0u), node_half(nd, 1u));
+        t.ref = (int)p;
+        t.height = max(t.height, height[2 * (size_t)p + (side ^ 1u)]) + 1u;
+        t.tris = nd.lcnt + nd.rcnt;
+        t.parent = up;
     }
 }
 
-__global__ void k_collapse_init(int2* __restrict__ list, unsigned int* __restrict__ counts) {
+// The nodes above the leaf tiles: a workgroup per group of 32 tiles, as far
+// as the nodes' indices are the group's (about ten subtrees a tile, one a
+// thread; one workgroup for all of them took 200 us at 1M triangles).
+constexpr int kTopBlock = 1024;
+__global__ __launch_bounds__(kTopBlock) void k_tree_groups(const uint32_t* __restrict__ parent, uint32_t ninner,
+                                                           BvhNode* nodes, uint32_t* arrived, uint32_t* height,
+                                                           const Pending* __restrict__ pending,
+                                                           Pending* __restrict__ top, uint32_t* __restrict__ cnt) {
+    const uint32_t first = blockIdx.x * (uint32_t)kGroupLeaves, last = min(first + (uint32_t)kGroupLeaves, ninner);
+    const uint32_t items = cnt[BC_COUNT + blockIdx.x];
+    const Pending* __restrict__ mine = pending + (size_t)blockIdx.x * kGroupTiles * kHandedOn;
+    for (uint32_t i = threadIdx.x; i < items; i += kTopBlock) {
+        Pending t = mine[i];
+        if (climb(t, first, last, parent, nodes, arrived, height)) top[atomicAdd(cnt + BC_TOP, 1u)] = t;
+    }
+}
+
+// The upper part of the tree in one workgroup: the binary nodes above the
+// groups, then the four-wide levels from the root down to the first with
+// kSubtrees nodes, which k_collapse takes over (or to the last). The levels'
+// lists alternate between the two queues; the final one is left in queue 0.
+constexpr uint32_t kSubtrees = 256;
+__global__ __launch_bounds__(kTopBlock) void k_tree_top(const uint32_t* __restrict__ parent, uint32_t ninner,
+                                                        BvhNode* nodes, uint32_t* arrived, uint32_t* height,
+                                                        const Pending* __restrict__ top, const uint32_t* __restrict__ ntop,
+                                                        Bvh4Node* __restrict__ nodes4, Open* __restrict__ queue,
+                                                        uint32_t* __restrict__ cnt) {
+    __shared__ Open level[2][4 * kSubtrees];
+    __shared__ uint32_t count[2];
+    const uint32_t items = *ntop;
+    for (uint32_t i = threadIdx.x; i < items; i += kTopBlock) {
+        Pending t = top[i];
+        if (climb(t, 0u, ninner, parent, nodes, arrived, height)) cnt[BC_DEPTH] = t.height;   // the root: one thread
+    }
     if (threadIdx.x == 0) {
-        list[0] = make_int2(0, 0);   // the binary root becomes four-wide node 0
-        counts[0] = 1u;              // level list A
-        counts[1] = 0u;              // level list B
-        counts[2] = 1u;              // four-wide nodes allocated
+        level[0][0] = Open{0u, 0, 1u};   // the binary root becomes four-wide node 0
+        count[0] = 1u;
+        count[1] = 0u;
     }
+    __syncthreads();
+    int cur = 0;
+    uint32_t n = 1;
+    while (n > 0u && n < kSubtrees) {
+        const bool live = threadIdx.x < n;
+        Open next[4];
+        const uint32_t inner = live ? collapse_node(level[cur][live ? threadIdx.x : 0u], nodes, nodes4, next) : 0u;
+        uint32_t sum;
+        const uint32_t below = wave_prefix4(inner, sum);
+        uint32_t base = 0;
+        if (__lane_id() == 0 && sum) base = atomicAdd(&count[cur ^ 1], sum);
+        base = __shfl(base, 0) + below;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e)
+            if (e < inner) level[cur ^ 1][base + e] = next[e];
+        __syncthreads();
+        n = count[cur ^ 1];
+        __syncthreads();
+        if (threadIdx.x == 0) count[cur] = 0u;
+        cur ^= 1;
+        __syncthreads();
+    }
+    for (uint32_t i = threadIdx.x; i < n; i += kTopBlock) queue[i] = level[cur][i];
+    if (threadIdx.x == 0) cnt[BC_QUEUE] = n;
 }
 
-__global__ void k_reset_count(unsigned int* __restrict__ c) {
-    if (threadIdx.x == 0) *c = 0u;
+// The subtrees of the nodes in `in`: every wave takes a run of them and works
+// through its own stack in LDS, up to 64 nodes at a time from the top.
+// Subtrees of one level differ in size by orders of magnitude, so a wave
+// stops after `budget` steps (0: none) and leaves what it still has in `out`,
+// which the next launch spreads over all waves again (1M triangles, 200
+// spheres: 860 us in one launch without a budget).
+// The stack: a step takes n nodes and pushes at most 4 n. Above kStackWide
+// entries a step takes a single node, so that the walk of the node on top
+// adds at most 3 entries per level (64) until it is done: with the 3 x 64 of
+// the last wide step never more than kStackSize.
+constexpr int kStackWide = 640, kStackSize = kStackWide + 2 * 3 * 64;
+constexpr int kCollapseWaves = 2048;
+constexpr int kCollapseBudget[kCollapseRounds] = {4, 8, 8, 0};
+__global__ __launch_bounds__(64) void k_collapse(const BvhNode* __restrict__ nodes, Bvh4Node* __restrict__ nodes4,
+                                                 uint32_t* __restrict__ cnt, int round, int budget, const Open* __restrict__ in, Open* __restrict__ out) {
+    __shared__ Open stack[kStackSize];
+    const uint32_t total = cnt[BC_QUEUE + round];
+    const uint32_t per = (total + gridDim.x - 1u) / gridDim.x;
+    uint32_t b = min(blockIdx.x * per, total);
+    const uint32_t e = min(b + per, total);
+    const int lane = __lane_id();
+    int sp = 0;
+    for (int step = 0; (sp > 0 || b < e) && (budget == 0 || step < budget); ++step) {
+        // lanes take nodes from the top of the stack, then from the wave's run
+        const int popped = sp > kStackWide ? 1 : min(sp, 64);
+        const int fresh = sp > kStackWide ? 0 : (int)min(e - b, (uint32_t)(64 - popped));
+        Open t{0u, 0, 0u};
+        if (lane < popped) t = stack[sp - 1 - lane];
+        else if (lane < popped + fresh) t = in[b + (uint32_t)(lane - popped)];
+        __syncthreads();   // one wave: its own order
+        Open next[4];
+        const uint32_t inner = lane < popped + fresh ? collapse_node(t, nodes, nodes4, next) : 0u;
+        sp -= popped;
+        b += (uint32_t)fresh;
+        uint32_t sum;
+        const uint32_t below = wave_prefix4(inner, sum);
+#pragma unroll
+        for (uint32_t q = 0; q < 4u; ++q)
+            if (q < inner) stack[sp + (int)(below + q)] = next[q];
+        sp += (int)sum;
+        __syncthreads();
+    }
+    if (sp == 0 && b >= e) return;
+    uint32_t o = 0;
+    if (lane == 0) o = atomicAdd(cnt + BC_QUEUE + round + 1, (uint32_t)sp + (e - b));
+    o = __shfl(o, 0);
+    for (int i = lane; i < sp; i += 64) out[o + (uint32_t)i] = stack[i];
+    o += (uint32_t)sp;
+    for (uint32_t i = b + (uint32_t)lane; i < e; i += 64u) out[o + (i - b)] = in[i];
 }
 
+// Quantised copies of all four-wide nodes (of the unused indices too: they are
+// never visited). On one node a lane takes as long as the collapse of a dozen
+// (forty divisions and search loops), so renders that traverse these nodes
+// make them, once per build or refit, and the others do not.
+__global__ __launch_bounds__(kBuildBlock) void k_quantise(const Bvh4Node* __restrict__ nodes4, uint32_t n,
+                                                          Bvh4QNode* __restrict__ nodes4q) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) nodes4q[i] = quantise_node(nodes4[i]);
+}
 
 inline size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -401,103 +623,90 @@ __global__ __launch_bounds__(kBuildBlock) void k_translate(float* __restrict__ p
 }
 
 // Scratch layout of a build over n triangles (kept after the build: the
-// sorted keys, the binary topology and the depth order are what a refit
-// reuses).
+// sorted keys and the parent links are what a refit reuses).
 struct BuildLayout {
-    size_t oBounds, oKeys, oKeys2, oChild, oParent, oIbox, oLbox, oDepth, oOrder, oLevels, oListA, oListB, oCounts,
-        oSort, sortBytes, total;
+    size_t groups, oBounds, oKeys, oKeys2, oParent, oArrived, oHeight, oPending, oTop, oQueue0, oQueue1, oCounts,
+        oSort, total;
 };
 
 hipError_t build_layout(rbh_ctx c, int n, BuildLayout& L) {
     const size_t nInt = n > 1 ? (size_t)n - 1 : 1;
+    L.groups = ((size_t)n + kGroupLeaves - 1) / kGroupLeaves;
+    const size_t tiles = ((size_t)n + kLeafTile - 1) / kLeafTile;
     size_t off = 0;
     L.oBounds = off; off = align_up(off + 64);
     L.oKeys = off; off = align_up(off + (size_t)n * 8);
     L.oKeys2 = off; off = align_up(off + (size_t)n * 8);
-    L.oChild = off; off = align_up(off + nInt * 8);
     L.oParent = off; off = align_up(off + ((size_t)n + nInt) * 4);
-    L.oIbox = off; off = align_up(off + nInt * 24);
-    L.oLbox = off; off = align_up(off + (size_t)n * 24);
-    L.oDepth = off; off = align_up(off + nInt * 4);
-    L.oOrder = off; off = align_up(off + nInt * 4);
-    L.oLevels = off; off = align_up(off + 3 * (kLevels + 1) * 4);
-    L.oListA = off; off = align_up(off + nInt * 8);
-    L.oListB = off; off = align_up(off + nInt * 8);
-    L.oCounts = off; off = align_up(off + 16);
-    L.sortBytes = std::max(radix::sort_scratch_bytes(n, 8, 0), radix::sort_scratch_bytes(nInt, 4, 4));
-    L.oSort = off; off = align_up(off + L.sortBytes);
+    L.oArrived = off; off = align_up(off + nInt * 4);
+    L.oHeight = off; off = align_up(off + nInt * 8);
+    L.oPending = off; off = align_up(off + tiles * kHandedOn * sizeof(Pending));
+    L.oTop = off; off = align_up(off + L.groups * kHandedOn * sizeof(Pending));
+    // nodes still to write: disjoint subtrees of at least two triangles
+    L.oQueue0 = off; off = align_up(off + ((size_t)n / 2 + 1) * sizeof(Open));
+    L.oQueue1 = off; off = align_up(off + ((size_t)n / 2 + 1) * sizeof(Open));
+    L.oCounts = off; off = align_up(off + (BC_COUNT + L.groups) * 4);
+    L.oSort = off; off = align_up(off + radix::sort_scratch_bytes(n, 8, 0));
     L.total = off;
     return hipSuccess;
 }
 
-int cu_count_of(int device) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) cus = 256;
-    return cus;
-}
-
 // The build's last stages, which a refit repeats over the kept topology:
-// leaf boxes and leaf-order triangle records from the current vertices,
-// internal boxes level by level, the two-child nodes and the four-wide
-// collapse.
+// triangle records and boxes from the current vertices, the two-child nodes
+// and the four-wide collapse.
 int build_boxes_and_nodes(rbh_ctx c, const BuildLayout& L) {
     Geometry& g = c->geom;
     Accel& acc = c->accel;
     const int n = (int)g.ntris;
-    const size_t nInt = n > 1 ? (size_t)n - 1 : 1;
     char* s = acc.scratch.as<char>();
     auto* keys2 = reinterpret_cast<unsigned long long*>(s + L.oKeys2);
-    int2* child = reinterpret_cast<int2*>(s + L.oChild);
-    float* ibox = reinterpret_cast<float*>(s + L.oIbox);
-    float* lbox = reinterpret_cast<float*>(s + L.oLbox);
-    int* order = reinterpret_cast<int*>(s + L.oOrder);
-    int* lstart = reinterpret_cast<int*>(s + L.oLevels);
-    const int nb = (n + kBuildBlock - 1) / kBuildBlock;
-    const int nbi = (int)((nInt + kBuildBlock - 1) / kBuildBlock);
-    const int cus = cu_count_of(c->device);
-    hipLaunchKernelGGL(k_leaves, dim3(nb), dim3(kBuildBlock), 0, c->stream, g.verts.as<float>(), g.indices.as<uint32_t>(),
-                       g.triMaterial.as<uint32_t>(), g.triLight.as<uint32_t>(), c->materials.as<Material>(),
-                       c->nmaterials, keys2, n, acc.keyIndexBits, lbox, acc.tris.as<TriRecord>());
+    auto* parent = reinterpret_cast<uint32_t*>(s + L.oParent);
+    auto* arrived = reinterpret_cast<uint32_t*>(s + L.oArrived);
+    auto* height = reinterpret_cast<uint32_t*>(s + L.oHeight);
+    auto* pending = reinterpret_cast<Pending*>(s + L.oPending);
+    auto* top = reinterpret_cast<Pending*>(s + L.oTop);
+    Open* queue[2] = {reinterpret_cast<Open*>(s + L.oQueue0), reinterpret_cast<Open*>(s + L.oQueue1)};
+    auto* cnt = reinterpret_cast<uint32_t*>(s + L.oCounts);
+    BvhNode* nodes = acc.nodes.as<BvhNode>();
+    Bvh4Node* nodes4 = acc.nodes4.as<Bvh4Node>();
+    const uint32_t ncnt = (uint32_t)(BC_COUNT + L.groups), ninner = (uint32_t)(n - 1);
+    hipLaunchKernelGGL(k_build_counters, dim3((ncnt + kBuildBlock - 1) / kBuildBlock), dim3(kBuildBlock), 0, c->stream, cnt,
+                       ncnt);
+    hipLaunchKernelGGL(k_leaves, dim3((n + kLeafTile - 1) / kLeafTile), dim3(kLeafBlock), 0, c->stream, g.verts.as<float>(),
+                       g.indices.as<uint32_t>(), g.triMaterial.as<uint32_t>(), g.triLight.as<uint32_t>(),
+                       c->materials.as<Material>(), c->nmaterials, keys2, n, acc.keyIndexBits, parent,
+                       acc.tris.as<TriRecord>(), nodes, arrived, height, pending, cnt);
     if (n > 1) {
-        const int lg = std::min(nbi, cus * 8);
-        for (int d = kLevels - 1; d >= 0; --d)
-            hipLaunchKernelGGL(k_refit_level, dim3(lg), dim3(kBuildBlock), 0, c->stream, d, lstart, order, child, ibox, lbox);
-        hipLaunchKernelGGL(k_emit, dim3(nbi), dim3(kBuildBlock), 0, c->stream, n, child, ibox, lbox, acc.nodes.as<BvhNode>());
-        int2* la = reinterpret_cast<int2*>(s + L.oListA);
-        int2* lb = reinterpret_cast<int2*>(s + L.oListB);
-        unsigned int* counts = reinterpret_cast<unsigned int*>(s + L.oCounts);
-        hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(64), 0, c->stream, la, counts);
-        // each level consumes one list and fills the other; every level
-        // descends at least one binary level, so 64 levels drain the tree
-        for (int lvl = 0; lvl < 64; ++lvl) {
-            const bool even = (lvl & 1) == 0;
-            unsigned int* inC = counts + (even ? 0 : 1);
-            unsigned int* outC = counts + (even ? 1 : 0);
-            hipLaunchKernelGGL(k_reset_count, dim3(1), dim3(64), 0, c->stream, outC);
-            hipLaunchKernelGGL(k_collapse, dim3(std::min(nbi, cus * 8)), dim3(kBuildBlock), 0, c->stream, child, ibox,
-                               lbox, even ? la : lb, inC, even ? lb : la, outC, counts + 2, acc.nodes4.as<Bvh4Node>(),
-                               acc.nodes4q.as<Bvh4QNode>());
-        }
+        // a single group's list is the top list
+        const bool one = L.groups == 1;
+        if (!one)
+            hipLaunchKernelGGL(k_tree_groups, dim3((unsigned)L.groups), dim3(kTopBlock), 0, c->stream, parent, ninner, nodes,
+                               arrived, height, pending, top, cnt);
+        hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(kTopBlock), 0, c->stream, parent, ninner, nodes, arrived, height,
+                           one ? pending : top, cnt + (one ? (int)BC_COUNT : (int)BC_TOP), nodes4, queue[0], cnt);
+        for (int r = 0; r < kCollapseRounds; ++r)
+            hipLaunchKernelGGL(k_collapse, dim3(kCollapseWaves), dim3(64), 0, c->stream, nodes, nodes4, cnt, r, kCollapseBudget[r],
+                               queue[r & 1], queue[(r & 1) ^ 1]);
     }
     RBH_HIP(c, hipGetLastError());
     return RBH_OK;
 }
 
-// Synchronises, times the stages since ev0 and checks the collapse.
-int finish_build(rbh_ctx c, const BuildLayout& L, float* ms) {
+// Synchronises, times the stages since ev0 and reads the depth.
+int finish_build(rbh_ctx c, const BuildLayout& L, float* ms, uint32_t* depth) {
     Accel& acc = c->accel;
     const int n = (int)c->geom.ntris;
-    const size_t nInt = n > 1 ? (size_t)n - 1 : 1;
     char* s = acc.scratch.as<char>();
     RBH_HIP(c, hipEventRecord(c->ev1, c->stream));
     RBH_HIP(c, hipStreamSynchronize(c->stream));
     RBH_HIP(c, hipEventElapsedTime(ms, c->ev0, c->ev1));
-    // counts: pending entries of both level lists, four-wide nodes allocated
-    uint32_t cnt4[3] = {0u, 0u, 0u};
-    if (n > 1) RBH_HIP(c, hipMemcpy(cnt4, s + L.oCounts, 12, hipMemcpyDeviceToHost));
-    if (n > 1 && (cnt4[0] != 0u || cnt4[2] > nInt))
-        return fail(c, RBH_ERR_RANGE, "four-wide collapse left %u nodes unwritten (%u allocated)", cnt4[0], cnt4[2]);
-    acc.nnodes4 = cnt4[2];
+    uint32_t cnt[BC_COUNT] = {};
+    if (n > 1) RBH_HIP(c, hipMemcpy(cnt, s + L.oCounts, sizeof(cnt), hipMemcpyDeviceToHost));
+    if (cnt[BC_QUEUE + kCollapseRounds] != 0u)
+        return fail(c, RBH_ERR_RANGE, "four-wide collapse left %u subtrees unwritten", cnt[BC_QUEUE + kCollapseRounds]);
+    acc.quantised = false;
+    acc.nnodes4 = n > 1 ? max_nodes4((uint32_t)n) : 0u;   // indices in use are below, with gaps
+    *depth = cnt[BC_DEPTH];
     return RBH_OK;
 }
 
@@ -513,25 +722,21 @@ int lbvh_build(rbh_ctx c) {
     RBH_ALLOC(c, acc.scratch, L.total);
     RBH_ALLOC(c, acc.nodes, nInt * sizeof(BvhNode));
     RBH_ALLOC(c, acc.tris, (size_t)n * sizeof(TriRecord));
-    RBH_ALLOC(c, acc.nodes4, nInt * sizeof(Bvh4Node));
-    RBH_ALLOC(c, acc.nodes4q, nInt * sizeof(Bvh4QNode));
+    const size_t n4 = std::max<size_t>(1, max_nodes4((uint32_t)n));
+    RBH_ALLOC(c, acc.nodes4, n4 * sizeof(Bvh4Node));
     char* s = acc.scratch.as<char>();
     acc.keysOffset = L.oKeys2;
     uint32_t* bounds = reinterpret_cast<uint32_t*>(s + L.oBounds);
     auto* keys = reinterpret_cast<unsigned long long*>(s + L.oKeys);
     auto* keys2 = reinterpret_cast<unsigned long long*>(s + L.oKeys2);
-    int2* child = reinterpret_cast<int2*>(s + L.oChild);
-    int* parent = reinterpret_cast<int*>(s + L.oParent);
-    int* ndepth = reinterpret_cast<int*>(s + L.oDepth);
-    int* order = reinterpret_cast<int*>(s + L.oOrder);
-    int* lstart = reinterpret_cast<int*>(s + L.oLevels);
 
     const float* v = g.verts.as<float>();
     const uint32_t* idx = g.indices.as<uint32_t>();
     const int nb = (n + kBuildBlock - 1) / kBuildBlock;
     RBH_HIP(c, hipEventRecord(c->ev0, c->stream));
     hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, c->stream, bounds);
-    hipLaunchKernelGGL(k_centroid_bounds, dim3(std::min(nb, 2048)), dim3(kBuildBlock), 0, c->stream, v, idx, (uint32_t)n, bounds);
+    hipLaunchKernelGGL(k_centroid_bounds, dim3(std::min(nb, kBoundsBlocks)), dim3(kBuildBlock), 0, c->stream, v, idx,
+                       (uint32_t)n, bounds);
     // key bits: the triangle index below, the Morton code above
     int idxBits = 1;
     while (idxBits < 32 && ((uint64_t)1 << idxBits) < (uint64_t)n) ++idxBits;
@@ -539,34 +744,18 @@ int lbvh_build(rbh_ctx c) {
     acc.keyIndexBits = idxBits;
     hipLaunchKernelGGL(k_morton, dim3(nb), dim3(kBuildBlock), 0, c->stream, v, idx, (uint32_t)n, bounds, axisBits,
                        idxBits, keys);
-    RBH_HIP(c, (radix::sort<unsigned long long, uint32_t>(s + L.oSort, keys, keys2, nullptr, nullptr, (uint32_t)n, 0, 64,
-                                                          c->stream)));
-    const int nbi = (int)((nInt + kBuildBlock - 1) / kBuildBlock);
-    if (n > 1) {
-        hipLaunchKernelGGL(k_karras, dim3(nbi), dim3(kBuildBlock), 0, c->stream, keys2, n, child, parent);
-        // internal nodes in depth order (list buffers are free until the collapse)
-        int2* ja = reinterpret_cast<int2*>(s + L.oListA);
-        int2* jb = reinterpret_cast<int2*>(s + L.oListB);
-        hipLaunchKernelGGL(k_jump_init, dim3(nbi), dim3(kBuildBlock), 0, c->stream, (int)nInt, parent, ja);
-        for (int r = 0; r < kJumpRounds; ++r) {
-            hipLaunchKernelGGL(k_jump, dim3(nbi), dim3(kBuildBlock), 0, c->stream, (int)nInt, ja, jb);
-            std::swap(ja, jb);
-        }
-        unsigned int* dkey = reinterpret_cast<unsigned int*>(ndepth);
-        int* ids = reinterpret_cast<int*>(jb);                       // free after the last round
-        unsigned int* dsorted = reinterpret_cast<unsigned int*>(ids + nInt);
-        hipLaunchKernelGGL(k_depth_keys, dim3(nbi), dim3(kBuildBlock), 0, c->stream, (int)nInt, ja, dkey, ids);
-        RBH_HIP(c, (radix::sort<unsigned int, int>(s + L.oSort, dkey, dsorted, ids, order, (uint32_t)nInt, 0, 7, c->stream)));
-        hipLaunchKernelGGL(k_level_bounds, dim3(1), dim3(128), 0, c->stream, dsorted, (int)nInt, lstart);
-    }
-    hipLaunchKernelGGL(k_depth, dim3(nb), dim3(kBuildBlock), 0, c->stream, n, parent, bounds + 6);
+    // stable, and the keys start in index order: sorting by the Morton bits sorts the keys
+    RBH_HIP(c, (radix::sort<unsigned long long, uint32_t>(s + L.oSort, keys, keys2, nullptr, nullptr, (uint32_t)n, idxBits,
+                                                          idxBits + 3 * axisBits, c->stream)));
+    if (n > 1)
+        hipLaunchKernelGGL(k_karras, dim3(((int)nInt + kBuildBlock - 1) / kBuildBlock), dim3(kBuildBlock), 0, c->stream,
+                           keys2, n, reinterpret_cast<uint32_t*>(s + L.oParent));
     const int rc = build_boxes_and_nodes(c, L);
     if (rc) return rc;
     float ms = 0.0f;
-    const int fr = finish_build(c, L, &ms);
-    if (fr) return fr;
     uint32_t depth = 0;
-    RBH_HIP(c, hipMemcpy(&depth, bounds + 6, 4, hipMemcpyDeviceToHost));
+    const int fr = finish_build(c, L, &ms, &depth);
+    if (fr) return fr;
     c->stats.bvhMs = ms;
     c->stats.bvhDepth = depth;
     acc.nnodes = n > 1 ? (uint32_t)(n - 1) : 0u;
@@ -575,6 +764,18 @@ int lbvh_build(rbh_ctx c) {
     if (depth > 64) return fail(c, RBH_ERR_RANGE, "LBVH depth %u exceeds the 64-entry traversal stack", depth);
     acc.built = true;
     acc.stale = false;
+    return RBH_OK;
+}
+
+int lbvh_quantise(rbh_ctx c, hipStream_t stream) {
+    Accel& acc = c->accel;
+    if (acc.quantised) return RBH_OK;
+    RBH_ALLOC(c, acc.nodes4q, std::max<size_t>(1, acc.nnodes4) * sizeof(Bvh4QNode));
+    if (acc.nnodes4 > 0)
+        hipLaunchKernelGGL(k_quantise, dim3((acc.nnodes4 + kBuildBlock - 1) / kBuildBlock), dim3(kBuildBlock), 0, stream,
+                           acc.nodes4.as<Bvh4Node>(), acc.nnodes4, acc.nodes4q.as<Bvh4QNode>());
+    RBH_HIP(c, hipGetLastError());
+    acc.quantised = true;
     return RBH_OK;
 }
 
@@ -606,7 +807,7 @@ hipError_t translate_points(rbh_ctx c, float* p, size_t npoints, uint32_t stride
 }
 
 // Refit: new vertex positions under the kept topology (the triangles' leaf
-// order, the binary hierarchy and its depth order stay; every box, the
+// order and the binary hierarchy stay; every box, the
 // triangle records and the four-wide nodes are recomputed). The traversal
 // stays exact for any positions; its cost grows as the positions drift from
 // the ones the hierarchy was built for.
@@ -622,7 +823,8 @@ int lbvh_refit(rbh_ctx c) {
     const int rc = build_boxes_and_nodes(c, L);
     if (rc) return rc;
     float ms = 0.0f;
-    const int fr = finish_build(c, L, &ms);
+    uint32_t depth = 0;
+    const int fr = finish_build(c, L, &ms, &depth);
     if (fr) return fr;
     c->stats.bvhMs = ms;
     acc.stale = false;

@@ -9,9 +9,11 @@
 // the four waves' digit counts are turned into bases in wave order in LDS, so
 // a key's place follows its index: the sort is stable. Across tiles, each
 // tile's digit counts are written digit-major (digit d of tile t at
-// d * tiles + t) and one exclusive scan turns them into every tile's first
-// output slot per digit. A pass is three launches: digit counts, scan,
-// ranked scatter; a sort is one pass per 8 key bits, ping-ponging between
+// d * tiles + t); one workgroup per digit scans its row and writes the row's
+// total, and the scatter scans the 256 totals for every digit's first slot
+// (one workgroup scanning all rows took 38 us a pass at 1M keys). A pass is
+// three launches: digit counts, row scans, ranked scatter; a sort is one pass
+// per 8 key bits, ping-ponging between
 // the output and a scratch buffer so that the last pass writes the output.
 // Compaction is the same with a one-bit digit: per-tile counts of selected
 // items, their scan (whose total is the number selected), ranked writes.
@@ -33,9 +35,9 @@ inline size_t tiles_for(size_t n) { return (n + kTile - 1) / kTile; }
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Scratch of a sort of n keys (and values, valBytes 0 without): the digit
-// counts, then the alternate key and value buffers.
+// counts and totals, then the alternate key and value buffers.
 inline size_t sort_scratch_bytes(size_t n, size_t keyBytes, size_t valBytes) {
-    return align256(tiles_for(n) * kBlock * 4) + align256(n * keyBytes) + align256(n * valBytes);
+    return align256((tiles_for(n) + 1) * kBlock * 4) + align256(n * keyBytes) + align256(n * valBytes);
 }
 // Scratch of a compaction of n items: the per-tile counts.
 inline size_t select_scratch_bytes(size_t n) { return align256(tiles_for(n) * 4 + 4); }
@@ -57,9 +59,10 @@ __global__ __launch_bounds__(kBlock) void k_digit_counts(const K* __restrict__ k
     counts[(size_t)threadIdx.x * tiles + blockIdx.x] = hist[threadIdx.x];
 }
 
-// Exclusive prefix sum of a[0..m) in place by one workgroup of B threads,
-// four consecutive elements per thread per round; *total (when given) = the
-// sum. (A template so that every translation unit may instantiate it.)
+// Exclusive prefix sum of a[0..m) in place by one workgroup of B threads
+// (of row blockIdx.x of m elements each), four consecutive elements per thread per round; *total (when given) = the
+// sum (total[row]). (A template so that every translation unit may
+// instantiate it.)
 template <int B>
 __global__ __launch_bounds__(B) void k_exclusive_scan(uint32_t* __restrict__ a, uint32_t m,
                                                       uint32_t* __restrict__ total) {
@@ -67,6 +70,7 @@ __global__ __launch_bounds__(B) void k_exclusive_scan(uint32_t* __restrict__ a, 
     __shared__ uint32_t wsum[W];
     const int lane = __lane_id(), w = (int)(threadIdx.x >> 6);
     uint32_t carry = 0u;
+    a += (size_t)blockIdx.x * m;
     for (uint32_t base = 0; base < m; base += B * 4) {
         const uint32_t j = base + threadIdx.x * 4;
         uint32_t v[4];
@@ -97,7 +101,7 @@ __global__ __launch_bounds__(B) void k_exclusive_scan(uint32_t* __restrict__ a, 
         carry += all;
         __syncthreads();   // wsum is rewritten next round
     }
-    if (total && threadIdx.x == 0) *total = carry;
+    if (total && threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
 // One pass of the sort: the keys (and values) of each tile to their slots.
@@ -105,12 +109,28 @@ template <typename K, typename VT, bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_ranked_scatter(const K* __restrict__ kin, K* __restrict__ kout,
                                                            const VT* __restrict__ vin, VT* __restrict__ vout,
                                                            uint32_t n, int shift, uint32_t mask,
-                                                           const uint32_t* __restrict__ offsets, uint32_t tiles) {
+                                                           const uint32_t* __restrict__ offsets,
+                                                           const uint32_t* __restrict__ totals, uint32_t tiles) {
     __shared__ uint32_t run[kBlock];
     __shared__ uint32_t wcnt[kWaves][kBlock];
     __shared__ uint32_t wbase[kWaves][kBlock];
     const int tid = (int)threadIdx.x, w = tid >> 6;
-    run[tid] = offsets[(size_t)tid * tiles + blockIdx.x];
+    {
+        // digit tid's first slot: the totals of the digits below it, then the tiles before this one
+        const uint32_t t = totals[tid];
+        uint32_t x = t;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = __shfl_up(x, o);
+            if (__lane_id() >= o) x += u;
+        }
+        if (__lane_id() == 63) wbase[0][w] = x;
+        __syncthreads();
+        uint32_t below = 0u;
+#pragma unroll
+        for (int k = 0; k < kWaves; ++k) below += k < w ? wbase[0][k] : 0u;
+        run[tid] = below + x - t + offsets[(size_t)tid * tiles + blockIdx.x];
+    }
 #pragma unroll
     for (int k = 0; k < kWaves; ++k) wcnt[k][tid] = 0u;
     __syncthreads();
@@ -165,7 +185,8 @@ hipError_t sort(void* scratch, const K* kin, K* kout, const VT* vin, VT* vout, u
     const uint32_t tiles = (uint32_t)tiles_for(n);
     char* p = static_cast<char*>(scratch);
     uint32_t* counts = reinterpret_cast<uint32_t*>(p);
-    K* altK = reinterpret_cast<K*>(p + align256((size_t)tiles * kBlock * 4));
+    uint32_t* totals = counts + (size_t)tiles * kBlock;
+    K* altK = reinterpret_cast<K*>(p + align256(((size_t)tiles + 1) * kBlock * 4));
     VT* altV = reinterpret_cast<VT*>(reinterpret_cast<char*>(altK) + align256((size_t)n * sizeof(K)));
     const int passes = (endBit - beginBit + 7) / 8;
     const K* src = kin;
@@ -178,14 +199,13 @@ hipError_t sort(void* scratch, const K* kin, K* kout, const VT* vin, VT* vout, u
         const int bits = endBit - shift < 8 ? endBit - shift : 8;
         const uint32_t mask = (1u << bits) - 1u;
         hipLaunchKernelGGL(k_digit_counts<K>, dim3(tiles), dim3(kBlock), 0, s, src, n, shift, mask, counts, tiles);
-        hipLaunchKernelGGL(k_exclusive_scan<kScanBlock>, dim3(1), dim3(kScanBlock), 0, s, counts, tiles * (uint32_t)kBlock,
-                           (uint32_t*)nullptr);
+        hipLaunchKernelGGL(k_exclusive_scan<kBlock>, dim3(kBlock), dim3(kBlock), 0, s, counts, tiles, totals);
         if (vin)
             hipLaunchKernelGGL((k_ranked_scatter<K, VT, true>), dim3(tiles), dim3(kBlock), 0, s, src, dst, vsrc, vdst,
-                               n, shift, mask, counts, tiles);
+                               n, shift, mask, counts, totals, tiles);
         else
             hipLaunchKernelGGL((k_ranked_scatter<K, VT, false>), dim3(tiles), dim3(kBlock), 0, s, src, dst, vsrc,
-                               vdst, n, shift, mask, counts, tiles);
+                               vdst, n, shift, mask, counts, totals, tiles);
         src = dst;
         vsrc = vdst;
     }

@@ -23,6 +23,9 @@
 #include "radix.hpp"
 
 namespace rbh {
+
+int lbvh_quantise(rbh_ctx c, hipStream_t stream);
+
 using namespace dev;
 namespace {
 
@@ -306,6 +309,11 @@ int rbh_test_trace(rbh_ctx c, const float* rays, float* hits, uint32_t n, int mo
     const uint32_t lanes = g.x * 128u;
     int* spill = (int*)s.out((size_t)lanes * kMaxStack4 * 4);
     STAGE_CHECK(dr && dh && spill);
+    if (mode & 8) {
+        const int rq = lbvh_quantise(c, c->stream);
+        if (rq) return rq;
+        RBH_HIP(c, hipStreamSynchronize(c->stream));
+    }
     const BvhNode* nodes = c->accel.nodes.as<BvhNode>();
     const Bvh4Node* nodes4 = c->accel.nodes4.as<Bvh4Node>();
     const Bvh4QNode* nodes4q = c->accel.nodes4q.as<Bvh4QNode>();

@@ -18,6 +18,7 @@ hipError_t resolve_launch(rbh_ctx c, const float* colorspace, float expo, void* 
 size_t trace_spill_words(size_t lanes);
 hipError_t light_tree_expand(rbh_ctx c);
 hipError_t refresh_tri_classes(rbh_ctx c);
+int lbvh_quantise(rbh_ctx c, hipStream_t stream);
 namespace host {
 int build_light_tree(const EmissiveTri* tris, const float* flux, uint32_t n, const ShapeLight* shapes,
                      const float* shapeFlux, uint32_t m, std::vector<PackedNode>& nodes,
@@ -621,6 +622,7 @@ int rbh_render(rbh_ctx c, const rbh_launch_params* lp) {
     const size_t NP = P * S;
     rc = prepare_accum(c, lp);
     if (rc) return rc;
+    if (rs.quantNodes && (rc = lbvh_quantise(c, c->stream)) != RBH_OK) return rc;
     Frame1 f{};
     fill_view(c, lp, f.sc);
     LaunchShape ls;
@@ -718,6 +720,10 @@ int rbh_render_batch(rbh_ctx owner, const rbh_ctx* scenes, const rbh_launch_para
                                               (unsigned long long)maxFilm);
     std::vector<SceneView> base(n);
     for (uint32_t s = 0; s < n; ++s) {
+        if (rs.quantNodes) {
+            const int rq = lbvh_quantise(scenes[s], owner->stream);
+            if (rq) return fail(owner, rq, "scene %u: %s", s, scenes[s]->err.c_str());
+        }
         fill_view(scenes[s], &lps[s], base[s]);
         // a scene may need fewer bounces than the pass runs; its paths end at its own caps
     }

@@ -1,0 +1,65 @@
+"""The LBVH's bottom-up boxes and four-wide collapse at the edges of their
+workgroups (2048 leaves a tile, 32 tiles a group), on even and on very uneven
+trees: node invariants over all nodes, the reported depth, and four-wide hits
+against the binary tree's, after a build and after a refit."""
+import numpy as np
+import pytest
+
+from test_lbvh_gpu import _rays, _read_lbvh, _trace, _upload
+
+pytestmark = pytest.mark.gpu
+
+
+def _triangles(n, spread, seed):
+    rng = np.random.default_rng(seed)
+    if spread == "even":
+        c = rng.uniform(-5, 5, (n, 3))
+    elif spread == "geometric":      # a cluster at every scale: the tree is deep on one side
+        c = np.exp2(-rng.uniform(0, 40, (n, 1))) * rng.uniform(0.5, 1.0, (n, 3)) * 10.0
+    else:                            # one centroid: the keys differ in the triangle index only
+        return np.tile(rng.normal(size=(3, 3)), (n, 1)).astype(np.float32)
+    return (c[:, None, :] + rng.normal(scale=0.05, size=(n, 3, 3))).reshape(-1, 3).astype(np.float32)
+
+
+def _check_tree(nodes, tris, n, depth):
+    lo = np.stack([nodes["lminx"], nodes["lminy"], nodes["lminz"]], 1), np.stack([nodes["rminx"], nodes["rminy"], nodes["rminz"]], 1)
+    hi = np.stack([nodes["lmaxx"], nodes["lmaxy"], nodes["lmaxz"]], 1), np.stack([nodes["rmaxx"], nodes["rmaxy"], nodes["rmaxz"]], 1)
+    ref = nodes["left"], nodes["right"]
+    tv = np.stack([tris["v0"], tris["v1"], tris["v2"]], 1)
+    for side in (0, 1):
+        inner = ref[side] >= 0
+        c = ref[side][inner]
+        assert np.array_equal(lo[side][inner], np.minimum(lo[0][c], lo[1][c]))
+        assert np.array_equal(hi[side][inner], np.maximum(hi[0][c], hi[1][c]))
+        t = ~ref[side][~inner]
+        assert np.array_equal(lo[side][~inner], tv[t].min(axis=1)) and np.array_equal(hi[side][~inner], tv[t].max(axis=1))
+    ch = np.concatenate(ref)
+    assert np.array_equal(np.sort(ch[ch >= 0]), np.arange(1, n - 1)) and np.array_equal(np.sort(~ch[ch < 0]), np.arange(n))
+    # levels from the root down; the last one with inner nodes is the leaves' depth
+    level, d = np.array([0]), 0
+    while len(level):
+        d += 1
+        level = np.concatenate([nodes["left"][level], nodes["right"][level]])
+        level = level[level >= 0]
+    assert d == depth
+
+
+@pytest.mark.parametrize("spread", ["even", "geometric", "one-centroid"])
+@pytest.mark.parametrize("n", [2, 3, 5, 2047, 2048, 2049, 2 * 2048 + 1, 65535, 65537, 3 * 65536 + 77])
+def test_tiles_and_groups(ctx, n, spread):
+    v = _triangles(n, spread, n)
+    idx = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    st = _upload(ctx, v, idx)
+    rays = _rays(np.random.default_rng(5), 500, -6, 6)
+    for refit in (False, True):
+        if refit:
+            v = (v * np.float32([1.0, -1.5, 0.75]) + np.float32(0.125)).astype(np.float32)
+            ctx.update_vertices(0, v)
+            ctx.refit_accel()
+        _, nodes, tris = _read_lbvh(ctx, n)
+        _check_tree(nodes, tris, n, st["bvhDepth"])
+        a, b = _trace(ctx, rays, False), _trace(ctx, rays, False, binary=True)
+        # the same closest distances; equal distances may name either triangle
+        assert np.array_equal(a[:, 0], b[:, 0])
+        q = _trace(ctx, rays, False, quant=True)
+        assert np.array_equal(a[:, 0], q[:, 0])
