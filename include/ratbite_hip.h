@@ -351,7 +351,7 @@ typedef struct rbh_tuning {
     int32_t shadeWaves;           /* shade-kernel register budget: 1 (unconstrained), 3 or 4 waves per SIMD */
     int32_t traceFetch;           /* 1: a trace/shadow lane takes a new ray as soon as its query completes; 0: waves take 64 rays at a time */
     int32_t traceWaves;           /* trace/shadow register budget (wave-synchronous kernels): 1 (unconstrained), 7 or 8 waves per SIMD */
-    int32_t quantNodes;           /* 1: the wave-synchronous trace/shadow kernels read the four-wide nodes quantised to 64 bytes */
+    int32_t quantNodes;           /* 1: the wave-synchronous trace/shadow kernels read the four-wide nodes with child boxes on an 11-bit grid (the default) */
     int32_t sortHits;             /* 1: material-sorted shading (hits queued by shading class: plain, transmissive and sheen
                                      ComplexSurface, PureConductor, PureDielectric, shape light) */
     double samplesPerSecond;      /* measured by rbh_autotune */

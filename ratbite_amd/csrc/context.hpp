@@ -78,8 +78,7 @@ struct Accel {
     uint32_t nnodes = 0, depth = 0;
     DevBuf nodes;     // BvhNode (binary LBVH)
     DevBuf nodes4;    // Bvh4Node (the binary tree collapsed four-wide; traversed)
-    DevBuf nodes4q;   // the four-wide nodes quantised to 64 bytes (Bvh4QNode), made when a render traverses them
-    bool quantised = false;
+    DevBuf nodes4h;   // the same nodes with boxes on an 11-bit grid (Bvh4HNode)
     uint32_t nnodes4 = 0;    // indices of four-wide nodes are below (with gaps)
     DevBuf tris;      // TriRecord in leaf order
     DevBuf scratch;   // build scratch
@@ -150,7 +149,7 @@ struct RenderState {
     int shadeWaves = 4;          // shade-kernel variant (1, 3, 4 waves per SIMD)
     int traceFetch = 0;          // 1: trace/shadow lanes fetch a new ray as soon as theirs completes
     int traceWaves = 7;          // trace/shadow register budget (1, 7, 8 waves per SIMD)
-    int quantNodes = 0;          // traverse the 64-byte quantised four-wide nodes
+    int quantNodes = 1;          // traverse the four-wide nodes with boxes on an 11-bit grid
     int sortHits = 1;            // shade conductor hits as their own run of the hit queue
     DevBuf sceneTable;           // batched passes: SceneView per scene and pass
     bool useGraph = false;       // replay each pass's launch sequence as a captured HIP graph

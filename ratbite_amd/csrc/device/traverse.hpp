@@ -11,22 +11,26 @@
 namespace rbh {
 namespace dev {
 
+// The ray's dominant axis and the shear that maps its direction to it. The
+// other two axes follow cyclically for either sign of the direction: swapping
+// them for a negative one, as published, negates U, V, W, the determinant and
+// T exactly, and the test makes the determinant positive anyway.
 struct RayShear {
-    int kx, ky, kz;
+    int kz;
     float Sx, Sy, Sz;
 };
-__device__ __forceinline__ float comp(V3 v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); }
+__device__ __forceinline__ V3 to_ray_axes(V3 v, int kz) {
+    const bool z = kz == 2, x = kz == 0;
+    return V3{z ? v.x : x ? v.y : v.z, z ? v.y : x ? v.z : v.x, z ? v.z : x ? v.x : v.y};
+}
 __device__ __forceinline__ RayShear make_shear(V3 d) {
     RayShear s;
     const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     s.kz = ax > ay ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
-    s.kx = s.kz == 2 ? 0 : s.kz + 1;
-    s.ky = s.kx == 2 ? 0 : s.kx + 1;
-    const float dz = comp(d, s.kz);
-    if (dz < 0.0f) { const int t = s.kx; s.kx = s.ky; s.ky = t; }
-    s.Sx = comp(d, s.kx) / dz;
-    s.Sy = comp(d, s.ky) / dz;
-    s.Sz = 1.0f / dz;
+    const V3 r = to_ray_axes(d, s.kz);
+    s.Sx = r.x / r.z;
+    s.Sy = r.y / r.z;
+    s.Sz = 1.0f / r.z;
     return s;
 }
 
@@ -42,13 +46,13 @@ __device__ __forceinline__ bool tri_candidate(const RayShear& s, V3 o, const Tri
     // No FMA contraction: the 2D edge functions of a shared edge must round
     // identically from both triangles for the test to stay watertight.
 #pragma clang fp contract(off)
-    const V3 A{tr.v0x - o.x, tr.v0y - o.y, tr.v0z - o.z};
-    const V3 B{tr.v1x - o.x, tr.v1y - o.y, tr.v1z - o.z};
-    const V3 C{tr.v2x - o.x, tr.v2y - o.y, tr.v2z - o.z};
-    const float Akz = comp(A, s.kz), Bkz = comp(B, s.kz), Ckz = comp(C, s.kz);
-    const float Ax = comp(A, s.kx) - s.Sx * Akz, Ay = comp(A, s.ky) - s.Sy * Akz;
-    const float Bx = comp(B, s.kx) - s.Sx * Bkz, By = comp(B, s.ky) - s.Sy * Bkz;
-    const float Cx = comp(C, s.kx) - s.Sx * Ckz, Cy = comp(C, s.ky) - s.Sy * Ckz;
+    const V3 A = to_ray_axes(V3{tr.v0x - o.x, tr.v0y - o.y, tr.v0z - o.z}, s.kz);
+    const V3 B = to_ray_axes(V3{tr.v1x - o.x, tr.v1y - o.y, tr.v1z - o.z}, s.kz);
+    const V3 C = to_ray_axes(V3{tr.v2x - o.x, tr.v2y - o.y, tr.v2z - o.z}, s.kz);
+    const float Akz = A.z, Bkz = B.z, Ckz = C.z;
+    const float Ax = A.x - s.Sx * Akz, Ay = A.y - s.Sy * Akz;
+    const float Bx = B.x - s.Sx * Bkz, By = B.y - s.Sy * Bkz;
+    const float Cx = C.x - s.Sx * Ckz, Cy = C.y - s.Sy * Ckz;
     float U = Cx * By - Cy * Bx, V = Ax * Cy - Ay * Cx, W = Bx * Ay - By * Ax;
     if (U == 0.0f || V == 0.0f || W == 0.0f) {
         U = (float)((double)Cx * By - (double)Cy * Bx);
@@ -96,6 +100,72 @@ struct TravStack {
     __device__ __forceinline__ int get(int sp) const {
         if (sp < LDS_DEPTH) return lds[sp * stride];
         return spill[(size_t)(sp - LDS_DEPTH) * spillStride];
+    }
+    // Pushes the children of the keys that are not ~0, the last one first.
+    // With room in the LDS part every child is written, a missing one where
+    // the next push overwrites it: no branch per child.
+    template <typename CHILD>
+    __device__ __forceinline__ void push3(int& sp, uint32_t k1, uint32_t k2, uint32_t k3, CHILD child) const {
+        if (sp + 3 <= LDS_DEPTH) {
+            lds[sp * stride] = child(k3);
+            sp += k3 != ~0u ? 1 : 0;
+            lds[sp * stride] = child(k2);
+            sp += k2 != ~0u ? 1 : 0;
+            lds[sp * stride] = child(k1);
+            sp += k1 != ~0u ? 1 : 0;
+        } else {
+            if (k3 != ~0u) put(sp++, child(k3));
+            if (k2 != ~0u) put(sp++, child(k2));
+            if (k1 != ~0u) put(sp++, child(k1));
+        }
+    }
+    __device__ __forceinline__ bool beyond(int, float) const { return false; }
+};
+
+// The same stack with the entry distance of each deferred subtree, its upper
+// 16 bits (rounded towards the ray's origin): a closest-hit walk drops the
+// entries that lie beyond the hit found since, instead of visiting them and
+// missing all their boxes. (Spilled entries have no distance and are visited.)
+template <int LDS_DEPTH>
+struct DistStack {
+    int* __restrict__ lds;
+    uint16_t* __restrict__ dist;
+    int stride;
+    int* __restrict__ spill;
+    uint32_t spillStride;
+    template <typename CHILD>
+    __device__ __forceinline__ void push3(int& sp, uint32_t k1, uint32_t k2, uint32_t k3, CHILD child) const {
+        if (sp + 3 <= LDS_DEPTH) {
+            lds[sp * stride] = child(k3);
+            dist[sp * stride] = (uint16_t)(k3 >> 16);
+            sp += k3 != ~0u ? 1 : 0;
+            lds[sp * stride] = child(k2);
+            dist[sp * stride] = (uint16_t)(k2 >> 16);
+            sp += k2 != ~0u ? 1 : 0;
+            lds[sp * stride] = child(k1);
+            dist[sp * stride] = (uint16_t)(k1 >> 16);
+            sp += k1 != ~0u ? 1 : 0;
+        } else {
+            if (k3 != ~0u) put(sp++, child(k3), k3);
+            if (k2 != ~0u) put(sp++, child(k2), k2);
+            if (k1 != ~0u) put(sp++, child(k1), k1);
+        }
+    }
+    __device__ __forceinline__ void put(int sp, int v, uint32_t key) const {
+        if (sp < LDS_DEPTH) {
+            lds[sp * stride] = v;
+            dist[sp * stride] = (uint16_t)(key >> 16);
+        } else {
+            spill[(size_t)(sp - LDS_DEPTH) * spillStride] = v;
+        }
+    }
+    __device__ __forceinline__ int get(int sp) const {
+        if (sp < LDS_DEPTH) return lds[sp * stride];
+        return spill[(size_t)(sp - LDS_DEPTH) * spillStride];
+    }
+    // the subtree of entry sp starts after distance `limit`
+    __device__ __forceinline__ bool beyond(int sp, float limit) const {
+        return sp < LDS_DEPTH && __uint_as_float((uint32_t)dist[sp * stride] << 16) > limit;
     }
 };
 
@@ -167,18 +237,31 @@ __device__ __forceinline__ Hit traverse(const BvhNode* __restrict__ nodes, const
 struct TravRay {
     V3 o, d;
     float ix, iy, iz;
+    uint32_t ox, oy, oz;   // byte offset in a Bvh4Node of the row of near planes per axis
     RayShear sh;
     Hit h;
     int node;   // next node to visit (~i: the root is triangle i)
     int sp;     // entries on the traversal stack
 };
 
+// 1 / d, or 1e30 if that is larger in size: a slab parallel to the ray is then
+// entered and left far away on either side, or never, without infinities times
+// zero. (Positive, so that a ray in a face meets the box on the grid: the
+// lower plane at exactly 0, the upper one at its margin of 2^-22.)
+__device__ __forceinline__ float finite_inverse(float d) {
+    const float i = 1.0f / d;
+    return fabsf(i) > 1e30f ? 1e30f : i;
+}
+
 __device__ __forceinline__ void trav_init(TravRay& r, V3 o, V3 d, float tmax, uint32_t nnodes) {
     r.o = o;
     r.d = d;
-    r.ix = 1.0f / d.x;
-    r.iy = 1.0f / d.y;
-    r.iz = 1.0f / d.z;
+    r.ix = finite_inverse(d.x);
+    r.iy = finite_inverse(d.y);
+    r.iz = finite_inverse(d.z);
+    r.ox = r.ix < 0.0f ? 16u : 0u;
+    r.oy = r.iy < 0.0f ? 48u : 32u;
+    r.oz = r.iz < 0.0f ? 80u : 64u;
     r.sh = make_shear(d);
     r.h.t = tmax;
     r.h.leaf = 0xFFFFFFFFu;
@@ -187,48 +270,104 @@ __device__ __forceinline__ void trav_init(TravRay& r, V3 o, V3 d, float tmax, ui
     r.sp = 0;
 }
 
-// Child boxes and references of one four-wide node.
-struct Box4 {
-    float lx[4], hx[4], ly[4], hy[4], lz[4], hz[4];
-    int ch[4];
+// A four-wide node as a ray meets it: where it enters and leaves the children's
+// boxes (not yet bounded by the ray's ends), and the child references.
+struct Visit4 {
+    float tn[4], tf[4];
+    uint32_t first;      // index of the first inner child
+    uint32_t order[4];   // inner children: their number among them; others: 4
+    uint32_t tris;       // slots with a triangle
 };
-__device__ __forceinline__ void load_node(const Bvh4Node* __restrict__ nodes, int i, Box4& b) {
-    const float4* q = reinterpret_cast<const float4*>(nodes + i);
-    const float4 lx = q[0], hx = q[1], ly = q[2], hy = q[3], lz = q[4], hz = q[5];
-    const int4 ch4 = reinterpret_cast<const int4*>(q)[6];
-    b.lx[0] = lx.x; b.lx[1] = lx.y; b.lx[2] = lx.z; b.lx[3] = lx.w;
-    b.hx[0] = hx.x; b.hx[1] = hx.y; b.hx[2] = hx.z; b.hx[3] = hx.w;
-    b.ly[0] = ly.x; b.ly[1] = ly.y; b.ly[2] = ly.z; b.ly[3] = ly.w;
-    b.hy[0] = hy.x; b.hy[1] = hy.y; b.hy[2] = hy.z; b.hy[3] = hy.w;
-    b.lz[0] = lz.x; b.lz[1] = lz.y; b.lz[2] = lz.z; b.lz[3] = lz.w;
-    b.hz[0] = hz.x; b.hz[1] = hz.y; b.hz[2] = hz.z; b.hz[3] = hz.w;
-    b.ch[0] = ch4.x; b.ch[1] = ch4.y; b.ch[2] = ch4.z; b.ch[3] = ch4.w;
-}
-__device__ __forceinline__ void load_node(const Bvh4QNode* __restrict__ nodes, int i, Box4& b) {
-    const uint4* q = reinterpret_cast<const uint4*>(nodes + i);
-    const uint4 h = q[0], c = q[1], a = q[2];
-    const uint2 e = reinterpret_cast<const uint2*>(q)[6];
-    const float ox = __uint_as_float(h.x), oy = __uint_as_float(h.y), oz = __uint_as_float(h.z);
-    const float sx = qnode_step(h.w & 0xFFu), sy = qnode_step((h.w >> 8) & 0xFFu), sz = qnode_step((h.w >> 16) & 0xFFu);
+// Of the two planes a box has on an axis the ray reaches the lower one first
+// if its direction is positive. Which row is the near one is an address here,
+// so the choice costs no instruction per child.
+__device__ __forceinline__ void visit_node(const Bvh4Node* __restrict__ nodes, const TravRay& r, Visit4& v) {
+    const char* base = reinterpret_cast<const char*>(nodes);
+    const uint32_t at = (uint32_t)r.node << 7;
+    auto row = [&](uint32_t off, float (&w)[4]) {
+        const float4 q = *reinterpret_cast<const float4*>(base + off);
+        w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+    };
+    float nx[4], fx[4], ny[4], fy[4], nz[4], fz[4];
+    row(at + r.ox, nx);
+    row((at + r.ox) ^ 16u, fx);
+    row(at + r.oy, ny);
+    row((at + r.oy) ^ 16u, fy);
+    row(at + r.oz, nz);
+    row((at + r.oz) ^ 16u, fz);
+    const int4 c4 = *reinterpret_cast<const int4*>(base + (at + 96u));
+    const uint32_t c[4] = {(uint32_t)c4.x, (uint32_t)c4.y, (uint32_t)c4.z, (uint32_t)c4.w};
+    // the inner children's indices are consecutive and the others have the sign bit
+    const uint32_t c01 = c[0] < c[1] ? c[0] : c[1], c23 = c[2] < c[3] ? c[2] : c[3];
+    v.first = c01 < c23 ? c01 : c23;
+    v.tris = 0u;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        b.lx[k] = qnode_decode(ox, (a.x >> (8 * k)) & 0xFFu, sx);
-        b.ly[k] = qnode_decode(oy, (a.y >> (8 * k)) & 0xFFu, sy);
-        b.lz[k] = qnode_decode(oz, (a.z >> (8 * k)) & 0xFFu, sz);
-        b.hx[k] = qnode_decode(ox, (a.w >> (8 * k)) & 0xFFu, sx);
-        b.hy[k] = qnode_decode(oy, (e.x >> (8 * k)) & 0xFFu, sy);
-        b.hz[k] = qnode_decode(oz, (e.y >> (8 * k)) & 0xFFu, sz);
+        v.tn[k] = fmaxf(fmaxf((nx[k] - r.o.x) * r.ix, (ny[k] - r.o.y) * r.iy), (nz[k] - r.o.z) * r.iz);
+        v.tf[k] = fminf(fminf((fx[k] - r.o.x) * r.ix, (fy[k] - r.o.y) * r.iy), (fz[k] - r.o.z) * r.iz);
+        v.order[k] = (int32_t)c[k] >= 0 ? c[k] - v.first : 4u;
+        v.tris |= c[k] > (uint32_t)kBvh4Empty ? 1u << k : 0u;
     }
-    b.ch[0] = (int)c.x; b.ch[1] = (int)c.y; b.ch[2] = (int)c.z; b.ch[3] = (int)c.w;
+}
+// On the grid plane q is met at q * (2^e / d) + (o - origin) / d: one fused
+// multiply-add per plane. The second term, computed with two roundings, is
+// moved outwards by four units of its own size (2^-22), which covers them and
+// the rounding of the product's factor; the relative error of the sum is the
+// caller's margin.
+__device__ __forceinline__ void visit_node(const Bvh4HNode* __restrict__ nodes, const TravRay& r, Visit4& v) {
+    const Bvh4HNode* __restrict__ nd = nodes + r.node;
+    const uint4* q = reinterpret_cast<const uint4*>(nd);
+    const uint4 h = q[0], rx = q[1], ry = q[2], rz = q[3];
+    v.first = (uint32_t)nd->child[0];
+    auto axis = [&](int sh, uint32_t ow, float o, float i, const uint4& w, float (&n)[4], float (&f)[4]) {
+        const float a = ldexpf(i, (int)(h.w << (24 - sh)) >> 24);
+        const float b = (__uint_as_float(ow) - o) * i;
+        const float bn = fmaf(fabsf(b), -2.3841858e-7f, b), bf = fmaf(fabsf(b), 2.3841858e-7f, b);
+        const bool neg = i < 0.0f;
+        const uint32_t n0 = neg ? w.z : w.x, n1 = neg ? w.w : w.y, f0 = neg ? w.x : w.z, f1 = neg ? w.y : w.w;
+        auto half = [](uint32_t u, int k) {
+            return (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> (16 * k)));
+        };
+        n[0] = fmaf(half(n0, 0), a, bn); n[1] = fmaf(half(n0, 1), a, bn);
+        n[2] = fmaf(half(n1, 0), a, bn); n[3] = fmaf(half(n1, 1), a, bn);
+        f[0] = fmaf(half(f0, 0), a, bf); f[1] = fmaf(half(f0, 1), a, bf);
+        f[2] = fmaf(half(f1, 0), a, bf); f[3] = fmaf(half(f1, 1), a, bf);
+    };
+    float nx[4], fx[4], ny[4], fy[4], nz[4], fz[4];
+    axis(0, h.x, r.o.x, r.ix, rx, nx, fx);
+    axis(8, h.y, r.o.y, r.iy, ry, ny, fy);
+    axis(16, h.z, r.o.z, r.iz, rz, nz, fz);
+    v.tris = (h.w >> 24) & 15u;
+    const uint32_t inner = h.w >> 28;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        v.tn[k] = fmaxf(fmaxf(nx[k], ny[k]), nz[k]);
+        v.tf[k] = fminf(fminf(fx[k], fy[k]), fz[k]);
+        v.order[k] = k < inner ? k : 4u;
+    }
+}
+
+__device__ __forceinline__ uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
+__device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a < b ? b : a; }
+__device__ __forceinline__ uint32_t med3_u(uint32_t a, uint32_t b, uint32_t c) {
+    return max_u(min_u(a, b), min_u(max_u(a, b), c));
 }
 
 // Visits r.node: tests its triangle children (nearest hit so far shortens
 // the ray), descends into the nearest box hit and defers the others,
 // nearest last on the stack. Returns true when the query is complete.
-// NODE: Bvh4Node or its 64-byte quantised form Bvh4QNode.
-template <bool ANY, int LDS_DEPTH, typename NODE>
+// NODE: Bvh4Node or Bvh4HNode.
+// The kernels that walk are bound by the latency of a step: waves wait for
+// memory in 60% of their cycles at 25 waves a CU, and a CU issues 0.85 vector
+// instructions a cycle (1.4 in k_accumulate). So a step loads little (68 bytes
+// instead of 112), its pushes and its sorting network have no branches, and
+// entries beyond the hit are dropped when they are popped. 1080p frame of 4.1M
+// triangles at 64 samples, against four rows a box, a branch per push and no
+// dropping: bounce rays 31.3 -> 25.8 ms, shadow rays 21.1 -> 16.6 ms, camera
+// rays 25.3 -> 25.0 ms.
+template <bool ANY, typename STACK, typename NODE>
 __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                          TravRay& r, const TravStack<LDS_DEPTH>& stack) {
+                                          TravRay& r, const STACK& stack) {
     if (r.node < 0) {
         // a single-triangle scene: the root is the leaf
         const TriRecord& tr = tris[~r.node];
@@ -241,25 +380,16 @@ __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const 
         }
         return true;
     }
-    Box4 bx;
-    load_node(nodes, r.node, bx);
-    const float* lxa = bx.lx; const float* hxa = bx.hx;
-    const float* lya = bx.ly; const float* hya = bx.hy;
-    const float* lza = bx.lz; const float* hza = bx.hz;
-    const int* cha = bx.ch;
+    Visit4 v;
+    visit_node(nodes, r, v);
     float tn[4];
     bool in[4];
     {
         const float best = r.h.t * 1.00000024f;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const float x0 = (lxa[k] - r.o.x) * r.ix, x1 = (hxa[k] - r.o.x) * r.ix;
-            const float y0 = (lya[k] - r.o.y) * r.iy, y1 = (hya[k] - r.o.y) * r.iy;
-            const float z0 = (lza[k] - r.o.z) * r.iz, z1 = (hza[k] - r.o.z) * r.iz;
-            const float tnear = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
-            const float tfar = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), best));
-            tn[k] = tnear;
-            in[k] = cha[k] != kBvh4Empty && tnear <= tfar * 1.00000024f;
+            tn[k] = fmaxf(v.tn[k], 0.0f);
+            in[k] = tn[k] <= fminf(v.tf[k], best) * 1.0000005f;
         }
     }
     // Triangle children first (a hit shortens the ray for the boxes), in
@@ -268,11 +398,12 @@ __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const 
     // of once for every slot in which some lane has one.
     uint32_t triMask = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) triMask |= (in[k] && cha[k] < 0) ? (1u << k) : 0u;
+    for (int k = 0; k < 4; ++k) triMask |= in[k] ? (1u << k) : 0u;
+    triMask &= v.tris;
     while (triMask) {
         const uint32_t k = (uint32_t)__builtin_ctz(triMask);
         triMask &= triMask - 1u;
-        const int c = k == 0u ? cha[0] : k == 1u ? cha[1] : k == 2u ? cha[2] : cha[3];
+        const int c = nodes[r.node].child[k];
         const TriRecord& tr = tris[~c];
         float t, b1, b2;
         if (tri_hit(r.sh, r.o, tr, r.h.t, t, b1, b2)) {
@@ -285,51 +416,41 @@ __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const 
     }
     // Surviving inner children nearest first. A child's key is the bit
     // pattern of its entry distance (>= 0, so ordered as an unsigned
-    // integer; the sign bit cleared for -0) with its slot in the two low bits, so a five-comparator
-    // network on unsigned min/max sorts them without branches or indexed
-    // registers; children within 4 ulp of each other go in slot order.
-    // Culled and empty slots sort last as ~0.
-    const float limit = r.h.t * 1.00000024f * 1.00000024f;
+    // integer; the sign bit cleared for -0) with its number among the node's
+    // inner children in the two low bits: their indices are consecutive, and
+    // children within 4 ulp of each other go in slot order. Culled and empty
+    // slots sort last as ~0.
+    const float limit = r.h.t * 1.00000024f * 1.0000005f;
     uint32_t key[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-        key[k] = (in[k] && cha[k] >= 0 && tn[k] <= limit) ? ((__float_as_uint(tn[k]) & 0x7FFFFFFCu) | (uint32_t)k)
-                                                          : ~0u;
-    {
-        auto cx = [](uint32_t& a, uint32_t& b) {
-            const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
-            a = lo;
-            b = hi;
-        };
-        cx(key[0], key[1]);
-        cx(key[2], key[3]);
-        cx(key[0], key[2]);
-        cx(key[1], key[3]);
-        cx(key[1], key[2]);
-    }
-    auto child = [&](uint32_t kk) {
-        const uint32_t s = kk & 3u;
-        return s == 0u ? cha[0] : s == 1u ? cha[1] : s == 2u ? cha[2] : cha[3];
-    };
-    if (key[0] != ~0u) {
+        key[k] = (in[k] && v.order[k] < 4u && (ANY || tn[k] <= limit)) ? ((__float_as_uint(tn[k]) & 0x7FFFFFFCu) | v.order[k])
+                                                                       : ~0u;
+    // three keys by minimum, median and maximum, the fourth inserted the same way
+    const uint32_t lo = min_u(min_u(key[0], key[1]), key[2]), mid = med3_u(key[0], key[1], key[2]),
+                   hi = max_u(max_u(key[0], key[1]), key[2]);
+    const uint32_t k0 = min_u(lo, key[3]), k1 = med3_u(lo, mid, key[3]), k2 = med3_u(mid, hi, key[3]), k3 = max_u(hi, key[3]);
+    auto child = [&](uint32_t kk) { return (int)(v.first + (kk & 3u)); };
+    if (k0 != ~0u) {
         // farthest pushed first, so the nearer ones are popped first
-        if (key[3] != ~0u) stack.put(r.sp++, child(key[3]));
-        if (key[2] != ~0u) stack.put(r.sp++, child(key[2]));
-        if (key[1] != ~0u) stack.put(r.sp++, child(key[1]));
-        r.node = child(key[0]);
+        stack.push3(r.sp, k1, k2, k3, child);
+        r.node = child(k0);
         return false;
     }
-    if (r.sp == 0) return true;
-    --r.sp;
-    r.node = stack.get(r.sp);
-    return false;
+    while (r.sp > 0) {
+        --r.sp;
+        if (!ANY && stack.beyond(r.sp, limit)) continue;
+        r.node = stack.get(r.sp);
+        return false;
+    }
+    return true;
 }
 
 // Whole query in one call: the closest hit below tmax or, with ANY, the
 // first one found.
-template <bool ANY, int LDS_DEPTH, typename NODE>
+template <bool ANY, typename STACK, typename NODE>
 __device__ __forceinline__ Hit traverse4(const NODE* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                         uint32_t nnodes, V3 o, V3 d, float tmax, const TravStack<LDS_DEPTH>& stack) {
+                                         uint32_t nnodes, V3 o, V3 d, float tmax, const STACK& stack) {
     TravRay r;
     trav_init(r, o, d, tmax, nnodes);
     while (!trav_step<ANY>(nodes, tris, r, stack)) {

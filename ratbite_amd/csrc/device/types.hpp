@@ -43,27 +43,24 @@ struct alignas(16) Bvh4Node {
     int32_t pad[4];
 };
 static_assert(sizeof(Bvh4Node) == 128, "Bvh4Node is 128 bytes");
+// The walks over them use 32-bit byte offsets; larger trees run the nodes below.
+constexpr uint32_t kMaxNodes4 = 1u << 25;
 
-// The same node quantised to 64 bytes: child boxes as 8-bit offsets from the
-// node's box corner o in power-of-two steps s per axis, decoded as
-// o + q * s (q * s is exact; one rounding in the add, the same in the builder
-// and in traversal, so the builder can make every decoded box contain its
-// child: lower bounds rounded down, upper bounds up).
-struct alignas(64) Bvh4QNode {
-    float ox, oy, oz;
-    uint32_t exps;                      // biased exponents of s: x bits 0-7, y 8-15, z 16-23
-    int32_t child[4];                   // as in Bvh4Node
-    uint32_t lox, loy, loz, hix;        // byte k = child k
-    uint32_t hiy, hiz;
-    uint32_t pad[2];
+// The same node with its child boxes on an 11-bit grid: plane q of an axis
+// lies at o + q * 2^e (exact arithmetic), o the lower corner of the boxes, and
+// every box on the grid contains its child. The grid coordinates are half
+// floats, integers that one fused multiply-add turns into a ray distance, so
+// that a visit loads 64 bytes and the first child's index instead of 112
+// bytes. Inner children come first, in slot order, then the triangles.
+struct alignas(128) Bvh4HNode {
+    float o[3];
+    uint32_t meta;           // e per axis as signed bytes (x lowest), bits 24-27 slots with a triangle, 28-30 number of inner children
+    uint16_t row[3][2][4];   // per axis: the lower planes of the four slots, the upper ones (half floats; empty slot: +inf, -inf)
+    int32_t child[4];        // as in Bvh4Node
+    int32_t pad[12];
 };
-static_assert(sizeof(Bvh4QNode) == 64, "Bvh4QNode is 64 bytes");
-__host__ __device__ inline float qnode_step(uint32_t expByte) {
-    union { uint32_t u; float f; } v;
-    v.u = expByte << 23;
-    return v.f;
-}
-__host__ __device__ inline float qnode_decode(float o, uint32_t q, float s) { return o + (float)q * s; }
+static_assert(sizeof(Bvh4HNode) == 128, "Bvh4HNode is 128 bytes");
+constexpr int kGridMax = 2047;
 
 // Triangle in leaf order, one 64-byte line: the vertices the traversal
 // tests (first 48 bytes), and what shading needs besides them: the original

@@ -64,7 +64,7 @@ struct SceneView {
     // geometry
     const BvhNode* nodes;
     const Bvh4Node* nodes4;
-    const Bvh4QNode* nodes4q;
+    const Bvh4HNode* nodes4h;
     const TriRecord* tris;
     uint32_t nnodes, nnodes4;
     const float* verts;
@@ -103,7 +103,8 @@ struct LaunchShape {
     int shadeWaves;          // register budget of the shade kernel: 1 (free), 3 or 4 waves per SIMD
     int traceFetch;          // trace/shadow lanes fetch a new ray when theirs completes (1) or wave by wave (0)
     int traceWaves;          // register budget of the wave-synchronous trace/shadow kernels: 1 (free), 7 or 8
-    int quantNodes;          // wave-synchronous trace/shadow kernels read the 64-byte quantised nodes
+    int quantNodes;          // wave-synchronous trace/shadow kernels read the nodes on an 11-bit grid
+    bool quantOnly;          // a tree of the pass is too large for the nodes with full boxes
     int sortHits;            // queue the hits by shading class (material-sorted shading)
 };
 

@@ -37,7 +37,11 @@ using namespace wf;
 
 namespace {
 
-constexpr int kStackLds = 16;   // traversal stack entries kept in LDS per lane
+// Traversal stack entries kept in LDS per lane: of the any-hit walk, and of
+// the closest-hit walk with their distances (6 bytes each), as many as leave
+// room for the seven waves per SIMD that the registers allow
+constexpr int kStackLds = 16;
+constexpr int kDistLds = 12;
 
 __device__ __forceinline__ uint32_t wave_push(uint32_t* __restrict__ counter, bool pred) {
     // one atomic per wave: ballot, leader adds the popcount, lanes take
@@ -149,6 +153,10 @@ __device__ __forceinline__ TravStack<kStackLds> lane_stack(const Frame1& f, int*
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     return TravStack<kStackLds>{lds + threadIdx.x, (int)blockDim.x, f.spill + t, f.spillStride};
 }
+__device__ __forceinline__ DistStack<kDistLds> lane_stack(const Frame1& f, int* lds, uint16_t* dist) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    return DistStack<kDistLds>{lds + threadIdx.x, dist + threadIdx.x, (int)blockDim.x, f.spill + t, f.spillStride};
+}
 
 // Wave-private staging of queue pushes: finished rays are appended to an
 // LDS list of the wave and written out 64 or more at a time with one atomic,
@@ -218,16 +226,16 @@ struct ClassList {
     }
 };
 
-// The four-wide nodes a kernel traverses: 128-byte or quantised 64-byte
+// The four-wide nodes a kernel traverses: full boxes or on an 11-bit grid
 template <bool QN>
 __device__ __forceinline__ auto scene_nodes(const SceneView& S) {
-    if constexpr (QN) return S.nodes4q;
+    if constexpr (QN) return S.nodes4h;
     else return S.nodes4;
 }
 
 // WAVES: minimum resident waves per SIMD the register allocation must allow
 // (1 = unconstrained), traded by the launch shape against spills; QN: the
-// quantised 64-byte nodes
+// nodes on an 11-bit grid
 // CAM0: the first bounce of a pass without depth of field, whose camera
 // rays all start at the camera position, the origin of the camera-relative
 // scene: the origin is the constant 0 there, which removes the origin
@@ -235,10 +243,11 @@ __device__ __forceinline__ auto scene_nodes(const SceneView& S) {
 // walk is the same).
 template <bool BATCH, bool FETCH, int WAVES, bool QN, bool CAM0>
 __global__ __launch_bounds__(kTraceBlock, WAVES) void k_trace(Frame1 f, uint32_t qsel) {
-    __shared__ int stack[kStackLds * kTraceBlock];
+    __shared__ int stack[kDistLds * kTraceBlock];
+    __shared__ uint16_t dist[kDistLds * kTraceBlock];
     __shared__ uint32_t staged[2 * kTraceBlock * 2];   // per wave: 128 hits, 128 misses
     __shared__ uint8_t stagedCls[2 * kTraceBlock];     // per wave: the hits' shading classes
-    const TravStack<kStackLds> st = lane_stack(f, stack);
+    const DistStack<kDistLds> st = lane_stack(f, stack, dist);
     const uint32_t count = f.counters[qsel ? CNT_QUEUE1 : CNT_QUEUE0];
     if (f.bounce > 0u && count <= f.tail) return;   // k_paths ran these paths to their end
     const uint32_t* __restrict__ queue = qsel ? f.p.q1 : f.p.q0;
@@ -572,7 +581,7 @@ hipError_t light_tree_expand(rbh_ctx c) {
 }
 
 // Spill entries per lane of the traversal stack beyond the LDS part.
-size_t trace_spill_words(size_t lanes) { return lanes * (size_t)(kMaxStack4 - kStackLds); }
+size_t trace_spill_words(size_t lanes) { return lanes * (size_t)(kMaxStack4 - kDistLds); }
 
 template <bool BATCH, bool FETCH, bool QN>
 static void launch_trace_q(rbh_ctx c, const Frame1& f, uint32_t qsel, const LaunchShape& ls) {
@@ -588,11 +597,12 @@ static void launch_trace_q(rbh_ctx c, const Frame1& f, uint32_t qsel, const Laun
     else hipLaunchKernelGGL((k_trace<BATCH, FETCH, 1, QN, false>), g, b, 0, c->stream, f, qsel);
 }
 
-// the work-fetch variants read the 128-byte nodes
+// The work-fetch variants read the nodes with full boxes, which are indexed
+// up to 4 GiB; larger trees run the nodes on the grid.
 template <bool BATCH>
 static void launch_trace(rbh_ctx c, const Frame1& f, uint32_t qsel, const LaunchShape& ls) {
-    if (ls.traceFetch) launch_trace_q<BATCH, true, false>(c, f, qsel, ls);
-    else if (ls.quantNodes) launch_trace_q<BATCH, false, true>(c, f, qsel, ls);
+    if (ls.traceFetch && !ls.quantOnly) launch_trace_q<BATCH, true, false>(c, f, qsel, ls);
+    else if (ls.quantNodes || ls.quantOnly) launch_trace_q<BATCH, false, true>(c, f, qsel, ls);
     else launch_trace_q<BATCH, false, false>(c, f, qsel, ls);
 }
 
@@ -606,8 +616,8 @@ static void launch_shadow_q(rbh_ctx c, const Frame1& f, const LaunchShape& ls) {
 
 template <bool BATCH>
 static void launch_shadow(rbh_ctx c, const Frame1& f, const LaunchShape& ls) {
-    if (ls.traceFetch) launch_shadow_q<BATCH, true, false>(c, f, ls);
-    else if (ls.quantNodes) launch_shadow_q<BATCH, false, true>(c, f, ls);
+    if (ls.traceFetch && !ls.quantOnly) launch_shadow_q<BATCH, true, false>(c, f, ls);
+    else if (ls.quantNodes || ls.quantOnly) launch_shadow_q<BATCH, false, true>(c, f, ls);
     else launch_shadow_q<BATCH, false, false>(c, f, ls);
 }
 

@@ -16,7 +16,8 @@
 //      nodes above (no cross-XCD fences: only kernel boundaries order the
 //      two). A node is emitted where its children meet, as the 64-byte
 //      two-child node with both child boxes
-//   6. collapse into 128-byte four-wide nodes, top down: a four-wide node
+//   6. collapse into 128-byte four-wide nodes (with full boxes and on an
+//      11-bit grid), top down: a four-wide node
 //      takes its binary node's children and keeps opening the inner child
 //      with the largest box surface until it has four. The same workgroup
 //      runs the upper levels, then one wave per subtree finishes. The inner
@@ -312,51 +313,40 @@ __device__ __forceinline__ float half_area(const Box& b) {
     return x * y + y * z + z * x;
 }
 
-// Biased exponent of the smallest power-of-two step s (s >= 2^-126) with
-// lo + 255 s >= hi in decode arithmetic.
-__device__ __forceinline__ uint32_t qnode_exponent(float lo, float hi) {
-    const float ext = hi - lo;
-    if (!(ext > 0.0f)) return 1u;
-    uint32_t e = (__float_as_uint(ext * (1.0f / 255.0f)) >> 23) & 0xFFu;
-    if (e == 0u) e = 1u;
-    while (e < 254u && qnode_decode(lo, 255u, qnode_step(e)) < hi) ++e;
-    return e;
-}
-// conservative 8-bit bounds of [clo, chi] on the grid lo + q s
-__device__ __forceinline__ void qnode_bounds(float lo, float s, float clo, float chi, uint32_t& qlo, uint32_t& qhi) {
-    qlo = (uint32_t)fminf(fmaxf(floorf((clo - lo) / s), 0.0f), 255.0f);
-    while (qlo > 0u && qnode_decode(lo, qlo, s) > clo) --qlo;
-    qhi = (uint32_t)fminf(fmaxf(ceilf((chi - lo) / s), 0.0f), 255.0f);
-    while (qhi < 255u && qnode_decode(lo, qhi, s) < chi) ++qhi;
-}
-
-// Quantised form of a four-wide node (empty slots get zero bytes; their
-// child reference masks them in traversal).
-__device__ __forceinline__ Bvh4QNode quantise_node(const Bvh4Node& nd) {
-    float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int k = 0; k < 4; ++k) {
-        if (nd.child[k] == kBvh4Empty) continue;
-        b[0] = fminf(b[0], nd.lox[k]); b[1] = fminf(b[1], nd.loy[k]); b[2] = fminf(b[2], nd.loz[k]);
-        b[3] = fmaxf(b[3], nd.hix[k]); b[4] = fmaxf(b[4], nd.hiy[k]); b[5] = fmaxf(b[5], nd.hiz[k]);
-    }
-    Bvh4QNode q;
-    q.ox = b[0]; q.oy = b[1]; q.oz = b[2];
-    const uint32_t ex = qnode_exponent(b[0], b[3]), ey = qnode_exponent(b[1], b[4]), ez = qnode_exponent(b[2], b[5]);
-    q.exps = ex | (ey << 8) | (ez << 16);
-    const float sx = qnode_step(ex), sy = qnode_step(ey), sz = qnode_step(ez);
-    q.lox = q.loy = q.loz = q.hix = q.hiy = q.hiz = 0u;
+// The 11-bit form of a four-wide node whose inner children come first. Grid
+// steps are powers of two and the arithmetic is in double precision, where a
+// difference of two floats divided by one is exact (or rounded by 2^-53, far
+// below the traversal's margin), so floor and ceil give planes outside.
+__device__ __forceinline__ Bvh4HNode grid_node(const Bvh4Node& nd) {
+    Bvh4HNode q;
+    uint32_t tris = 0u, inner = 0u;
+#pragma unroll
     for (int k = 0; k < 4; ++k) {
         q.child[k] = nd.child[k];
-        if (nd.child[k] == kBvh4Empty) continue;
-        uint32_t l, h;
-        qnode_bounds(b[0], sx, nd.lox[k], nd.hix[k], l, h);
-        q.lox |= l << (8 * k); q.hix |= h << (8 * k);
-        qnode_bounds(b[1], sy, nd.loy[k], nd.hiy[k], l, h);
-        q.loy |= l << (8 * k); q.hiy |= h << (8 * k);
-        qnode_bounds(b[2], sz, nd.loz[k], nd.hiz[k], l, h);
-        q.loz |= l << (8 * k); q.hiz |= h << (8 * k);
+        tris |= nd.child[k] < 0 && nd.child[k] != kBvh4Empty ? 1u << k : 0u;
+        inner += nd.child[k] >= 0 ? 1u : 0u;
     }
-    q.pad[0] = q.pad[1] = 0u;
+    q.meta = tris << 24 | inner << 28;
+    auto axis = [&](int a, const float (&lo)[4], const float (&hi)[4]) {
+        // empty boxes are (+inf, -inf)
+        const float o = fminf(fminf(lo[0], lo[1]), fminf(lo[2], lo[3])), top = fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3]));
+        int e = 0;
+        (void)frexp(((double)top - (double)o) / (double)kGridMax, &e);   // extent / 2047 < 2^e
+        e = min(max(e, -126), 127);
+        q.o[a] = o;
+        q.meta |= ((uint32_t)e & 0xFFu) << (8 * a);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double l = floor(ldexp((double)lo[k] - (double)o, -e)), h = ceil(ldexp((double)hi[k] - (double)o, -e));
+            q.row[a][0][k] = __builtin_bit_cast(uint16_t, (_Float16)(float)l);
+            q.row[a][1][k] = __builtin_bit_cast(uint16_t, (_Float16)(float)h);
+        }
+    };
+    axis(0, nd.lox, nd.hix);
+    axis(1, nd.loy, nd.hiy);
+    axis(2, nd.loz, nd.hiz);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) q.pad[k] = 0;
     return q;
 }
 
@@ -382,7 +372,7 @@ struct Open {
 // t.room + 1, ... in slot order, their subtrees' indices follow. Returns the
 // number of inner children, next[0..] the nodes to write for them.
 __device__ __forceinline__ uint32_t collapse_node(const Open& t, const BvhNode* nodes, Bvh4Node* __restrict__ nodes4,
-                                                  Open (&next)[4]) {
+                                                  Bvh4HNode* __restrict__ nodes4h, Open (&next)[4]) {
     Box box[4];
     int ref[4];
     uint32_t tris[4];
@@ -424,28 +414,41 @@ __device__ __forceinline__ uint32_t collapse_node(const Open& t, const BvhNode* 
         ref[ns] = nd.right;
         tris[ns] = nd.rcnt;
     }
+    // inner children first, either kind in its order
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass)
+#pragma unroll
+        for (int k = 0; k < 3 - pass; ++k)
+            if (ref[k] < 0 && ref[k + 1] >= 0) {
+                const Box b = box[k];
+                box[k] = box[k + 1];
+                box[k + 1] = b;
+                const int rf = ref[k];
+                ref[k] = ref[k + 1];
+                ref[k + 1] = rf;
+                const uint32_t tr = tris[k];
+                tris[k] = tris[k + 1];
+                tris[k + 1] = tr;
+            }
     uint32_t inner = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) inner += ref[k] >= 0 ? 1u : 0u;
     Bvh4Node out;
-    uint32_t id = t.room, room = t.room + inner, q = 0;
+    uint32_t id = t.room, room = t.room + inner;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         out.lox[k] = box[k].lo[0]; out.loy[k] = box[k].lo[1]; out.loz[k] = box[k].lo[2];
         out.hix[k] = box[k].hi[0]; out.hiy[k] = box[k].hi[1]; out.hiz[k] = box[k].hi[2];
         out.child[k] = ref[k];
         if (ref[k] >= 0) {
-            const Open o{id, ref[k], room};
+            next[k] = Open{id, ref[k], room};
             out.child[k] = (int)id++;
             room += max_nodes4(tris[k]) - 1u;
-#pragma unroll
-            for (uint32_t e = 0; e <= (uint32_t)k; ++e)
-                if (e == q) next[e] = o;
-            ++q;
         }
     }
     out.pad[0] = out.pad[1] = out.pad[2] = out.pad[3] = 0;
     nodes4[t.id] = out;
+    nodes4h[t.id] = grid_node(out);
     return inner;
 }
 
@@ -505,7 +508,8 @@ constexpr uint32_t kSubtrees = 256;
 __global__ __launch_bounds__(kTopBlock) void k_tree_top(const uint32_t* __restrict__ parent, uint32_t ninner,
                                                         BvhNode* nodes, uint32_t* arrived, uint32_t* height,
                                                         const Pending* __restrict__ top, const uint32_t* __restrict__ ntop,
-                                                        Bvh4Node* __restrict__ nodes4, Open* __restrict__ queue,
+                                                        Bvh4Node* __restrict__ nodes4,
+                                                        Bvh4HNode* __restrict__ nodes4h, Open* __restrict__ queue,
                                                         uint32_t* __restrict__ cnt) {
     __shared__ Open level[2][4 * kSubtrees];
     __shared__ uint32_t count[2];
@@ -525,7 +529,7 @@ __global__ __launch_bounds__(kTopBlock) void k_tree_top(const uint32_t* __restri
     while (n > 0u && n < kSubtrees) {
         const bool live = threadIdx.x < n;
         Open next[4];
-        const uint32_t inner = live ? collapse_node(level[cur][live ? threadIdx.x : 0u], nodes, nodes4, next) : 0u;
+        const uint32_t inner = live ? collapse_node(level[cur][live ? threadIdx.x : 0u], nodes, nodes4, nodes4h, next) : 0u;
         uint32_t sum;
         const uint32_t below = wave_prefix4(inner, sum);
         uint32_t base = 0;
@@ -559,7 +563,8 @@ constexpr int kStackWide = 640, kStackSize = kStackWide + 2 * 3 * 64;
 constexpr int kCollapseWaves = 2048;
 constexpr int kCollapseBudget[kCollapseRounds] = {4, 8, 8, 0};
 __global__ __launch_bounds__(64) void k_collapse(const BvhNode* __restrict__ nodes, Bvh4Node* __restrict__ nodes4,
-                                                 uint32_t* __restrict__ cnt, int round, int budget, const Open* __restrict__ in, Open* __restrict__ out) {
+                                                 Bvh4HNode* __restrict__ nodes4h, uint32_t* __restrict__ cnt, int round,
+                                                 int budget, const Open* __restrict__ in, Open* __restrict__ out) {
     __shared__ Open stack[kStackSize];
     const uint32_t total = cnt[BC_QUEUE + round];
     const uint32_t per = (total + gridDim.x - 1u) / gridDim.x;
@@ -576,7 +581,7 @@ __global__ __launch_bounds__(64) void k_collapse(const BvhNode* __restrict__ nod
         else if (lane < popped + fresh) t = in[b + (uint32_t)(lane - popped)];
         __syncthreads();   // one wave: its own order
         Open next[4];
-        const uint32_t inner = lane < popped + fresh ? collapse_node(t, nodes, nodes4, next) : 0u;
+        const uint32_t inner = lane < popped + fresh ? collapse_node(t, nodes, nodes4, nodes4h, next) : 0u;
         sp -= popped;
         b += (uint32_t)fresh;
         uint32_t sum;
@@ -594,16 +599,6 @@ __global__ __launch_bounds__(64) void k_collapse(const BvhNode* __restrict__ nod
     for (int i = lane; i < sp; i += 64) out[o + (uint32_t)i] = stack[i];
     o += (uint32_t)sp;
     for (uint32_t i = b + (uint32_t)lane; i < e; i += 64u) out[o + (i - b)] = in[i];
-}
-
-// Quantised copies of all four-wide nodes (of the unused indices too: they are
-// never visited). On one node a lane takes as long as the collapse of a dozen
-// (forty divisions and search loops), so renders that traverse these nodes
-// make them, once per build or refit, and the others do not.
-__global__ __launch_bounds__(kBuildBlock) void k_quantise(const Bvh4Node* __restrict__ nodes4, uint32_t n,
-                                                          Bvh4QNode* __restrict__ nodes4q) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) nodes4q[i] = quantise_node(nodes4[i]);
 }
 
 inline size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -669,6 +664,7 @@ int build_boxes_and_nodes(rbh_ctx c, const BuildLayout& L) {
     auto* cnt = reinterpret_cast<uint32_t*>(s + L.oCounts);
     BvhNode* nodes = acc.nodes.as<BvhNode>();
     Bvh4Node* nodes4 = acc.nodes4.as<Bvh4Node>();
+    Bvh4HNode* nodes4h = acc.nodes4h.as<Bvh4HNode>();
     const uint32_t ncnt = (uint32_t)(BC_COUNT + L.groups), ninner = (uint32_t)(n - 1);
     hipLaunchKernelGGL(k_build_counters, dim3((ncnt + kBuildBlock - 1) / kBuildBlock), dim3(kBuildBlock), 0, c->stream, cnt,
                        ncnt);
@@ -683,10 +679,10 @@ int build_boxes_and_nodes(rbh_ctx c, const BuildLayout& L) {
             hipLaunchKernelGGL(k_tree_groups, dim3((unsigned)L.groups), dim3(kTopBlock), 0, c->stream, parent, ninner, nodes,
                                arrived, height, pending, top, cnt);
         hipLaunchKernelGGL(k_tree_top, dim3(1), dim3(kTopBlock), 0, c->stream, parent, ninner, nodes, arrived, height,
-                           one ? pending : top, cnt + (one ? (int)BC_COUNT : (int)BC_TOP), nodes4, queue[0], cnt);
+                           one ? pending : top, cnt + (one ? (int)BC_COUNT : (int)BC_TOP), nodes4, nodes4h, queue[0], cnt);
         for (int r = 0; r < kCollapseRounds; ++r)
-            hipLaunchKernelGGL(k_collapse, dim3(kCollapseWaves), dim3(64), 0, c->stream, nodes, nodes4, cnt, r, kCollapseBudget[r],
-                               queue[r & 1], queue[(r & 1) ^ 1]);
+            hipLaunchKernelGGL(k_collapse, dim3(kCollapseWaves), dim3(64), 0, c->stream, nodes, nodes4, nodes4h, cnt, r,
+                               kCollapseBudget[r], queue[r & 1], queue[(r & 1) ^ 1]);
     }
     RBH_HIP(c, hipGetLastError());
     return RBH_OK;
@@ -704,7 +700,6 @@ int finish_build(rbh_ctx c, const BuildLayout& L, float* ms, uint32_t* depth) {
     if (n > 1) RBH_HIP(c, hipMemcpy(cnt, s + L.oCounts, sizeof(cnt), hipMemcpyDeviceToHost));
     if (cnt[BC_QUEUE + kCollapseRounds] != 0u)
         return fail(c, RBH_ERR_RANGE, "four-wide collapse left %u subtrees unwritten", cnt[BC_QUEUE + kCollapseRounds]);
-    acc.quantised = false;
     acc.nnodes4 = n > 1 ? max_nodes4((uint32_t)n) : 0u;   // indices in use are below, with gaps
     *depth = cnt[BC_DEPTH];
     return RBH_OK;
@@ -724,6 +719,7 @@ int lbvh_build(rbh_ctx c) {
     RBH_ALLOC(c, acc.tris, (size_t)n * sizeof(TriRecord));
     const size_t n4 = std::max<size_t>(1, max_nodes4((uint32_t)n));
     RBH_ALLOC(c, acc.nodes4, n4 * sizeof(Bvh4Node));
+    RBH_ALLOC(c, acc.nodes4h, n4 * sizeof(Bvh4HNode));
     char* s = acc.scratch.as<char>();
     acc.keysOffset = L.oKeys2;
     uint32_t* bounds = reinterpret_cast<uint32_t*>(s + L.oBounds);
@@ -764,18 +760,6 @@ int lbvh_build(rbh_ctx c) {
     if (depth > 64) return fail(c, RBH_ERR_RANGE, "LBVH depth %u exceeds the 64-entry traversal stack", depth);
     acc.built = true;
     acc.stale = false;
-    return RBH_OK;
-}
-
-int lbvh_quantise(rbh_ctx c, hipStream_t stream) {
-    Accel& acc = c->accel;
-    if (acc.quantised) return RBH_OK;
-    RBH_ALLOC(c, acc.nodes4q, std::max<size_t>(1, acc.nnodes4) * sizeof(Bvh4QNode));
-    if (acc.nnodes4 > 0)
-        hipLaunchKernelGGL(k_quantise, dim3((acc.nnodes4 + kBuildBlock - 1) / kBuildBlock), dim3(kBuildBlock), 0, stream,
-                           acc.nodes4.as<Bvh4Node>(), acc.nnodes4, acc.nodes4q.as<Bvh4QNode>());
-    RBH_HIP(c, hipGetLastError());
-    acc.quantised = true;
     return RBH_OK;
 }
 

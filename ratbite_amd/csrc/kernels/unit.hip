@@ -24,8 +24,6 @@
 
 namespace rbh {
 
-int lbvh_quantise(rbh_ctx c, hipStream_t stream);
-
 using namespace dev;
 namespace {
 
@@ -80,7 +78,7 @@ __global__ void k_oct(const float* v, uint32_t* enc, float* dec, uint32_t n) {
 
 template <bool ANY, int LDS_DEPTH>
 __global__ __launch_bounds__(128) void k_trace_test(const BvhNode* nodes, const Bvh4Node* nodes4,
-                                                    const Bvh4QNode* nodes4q, const TriRecord* tris, uint32_t nnodes,
+                                                    const Bvh4HNode* nodes4h, const TriRecord* tris, uint32_t nnodes,
                                                     uint32_t nnodes4, int tree, const float* rays, float* hits,
                                                     uint32_t n, int* spill, uint32_t spillStride) {
     __shared__ int stack[LDS_DEPTH * 128];
@@ -90,7 +88,7 @@ __global__ __launch_bounds__(128) void k_trace_test(const BvhNode* nodes, const 
     const float* r = rays + 8 * (size_t)i;
     const V3 ro{r[0], r[1], r[2]}, rd{r[4], r[5], r[6]};
     const Hit h = tree == 1 ? traverse<ANY>(nodes, tris, nnodes, ro, rd, r[7], st)
-                : tree == 2 ? traverse4<ANY>(nodes4q, tris, nnodes4, ro, rd, r[7], st)
+                : tree == 2 ? traverse4<ANY>(nodes4h, tris, nnodes4, ro, rd, r[7], st)
                             : traverse4<ANY>(nodes4, tris, nnodes4, ro, rd, r[7], st);
     float* o = hits + 4 * (size_t)i;
     o[0] = h.leaf == 0xFFFFFFFFu ? -1.0f : h.t;
@@ -309,14 +307,9 @@ int rbh_test_trace(rbh_ctx c, const float* rays, float* hits, uint32_t n, int mo
     const uint32_t lanes = g.x * 128u;
     int* spill = (int*)s.out((size_t)lanes * kMaxStack4 * 4);
     STAGE_CHECK(dr && dh && spill);
-    if (mode & 8) {
-        const int rq = lbvh_quantise(c, c->stream);
-        if (rq) return rq;
-        RBH_HIP(c, hipStreamSynchronize(c->stream));
-    }
     const BvhNode* nodes = c->accel.nodes.as<BvhNode>();
     const Bvh4Node* nodes4 = c->accel.nodes4.as<Bvh4Node>();
-    const Bvh4QNode* nodes4q = c->accel.nodes4q.as<Bvh4QNode>();
+    const Bvh4HNode* nodes4h = c->accel.nodes4h.as<Bvh4HNode>();
     const TriRecord* tris = c->accel.tris.as<TriRecord>();
     const uint32_t nn = c->accel.nnodes, nn4 = c->accel.nnodes4;
     const bool any = (mode & 1) != 0, tiny = (mode & 2) != 0;
@@ -335,15 +328,15 @@ int rbh_test_trace(rbh_ctx c, const float* rays, float* hits, uint32_t n, int mo
     const int binary = (mode & 4) ? 1 : ((mode & 8) ? 2 : 0);
     // mode bit 1: a 2-entry LDS stack, so the spill columns carry the rest;
     // bit 2: the binary tree instead of the four-wide one; bit 3: the
-    // four-wide nodes quantised to 64 bytes
+    // four-wide nodes on an 11-bit grid
     if (any && tiny)
-        hipLaunchKernelGGL((k_trace_test<true, 2>), g, dim3(128), 0, 0, nodes, nodes4, nodes4q, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
+        hipLaunchKernelGGL((k_trace_test<true, 2>), g, dim3(128), 0, 0, nodes, nodes4, nodes4h, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
     else if (any)
-        hipLaunchKernelGGL((k_trace_test<true, 16>), g, dim3(128), 0, 0, nodes, nodes4, nodes4q, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
+        hipLaunchKernelGGL((k_trace_test<true, 16>), g, dim3(128), 0, 0, nodes, nodes4, nodes4h, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
     else if (tiny)
-        hipLaunchKernelGGL((k_trace_test<false, 2>), g, dim3(128), 0, 0, nodes, nodes4, nodes4q, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
+        hipLaunchKernelGGL((k_trace_test<false, 2>), g, dim3(128), 0, 0, nodes, nodes4, nodes4h, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
     else
-        hipLaunchKernelGGL((k_trace_test<false, 16>), g, dim3(128), 0, 0, nodes, nodes4, nodes4q, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
+        hipLaunchKernelGGL((k_trace_test<false, 16>), g, dim3(128), 0, 0, nodes, nodes4, nodes4h, tris, nn, nn4, binary, (const float*)dr, (float*)dh, n, spill, lanes);
     FINISH(hits, dh, (size_t)n * 16);
     return RBH_OK;
 }

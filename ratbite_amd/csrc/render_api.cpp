@@ -18,7 +18,6 @@ hipError_t resolve_launch(rbh_ctx c, const float* colorspace, float expo, void* 
 size_t trace_spill_words(size_t lanes);
 hipError_t light_tree_expand(rbh_ctx c);
 hipError_t refresh_tri_classes(rbh_ctx c);
-int lbvh_quantise(rbh_ctx c, hipStream_t stream);
 namespace host {
 int build_light_tree(const EmissiveTri* tris, const float* flux, uint32_t n, const ShapeLight* shapes,
                      const float* shapeFlux, uint32_t m, std::vector<PackedNode>& nodes,
@@ -457,7 +456,7 @@ void fill_view(rbh_ctx c, const rbh_launch_params* lp, SceneView& v) {
     v.focus = lp->focusDistance;
     v.nodes = c->accel.nodes.as<BvhNode>();
     v.nodes4 = c->accel.nodes4.as<Bvh4Node>();
-    v.nodes4q = c->accel.nodes4q.as<Bvh4QNode>();
+    v.nodes4h = c->accel.nodes4h.as<Bvh4HNode>();
     v.nnodes4 = c->accel.nnodes4;
     v.tris = c->accel.tris.as<TriRecord>();
     v.nnodes = c->accel.nnodes;
@@ -514,6 +513,7 @@ int prepare_pass_state(rbh_ctx c, size_t NP, Frame1& f, LaunchShape& ls) {
     ls.traceFetch = rs.traceFetch;
     ls.traceWaves = rs.traceWaves;
     ls.quantNodes = rs.quantNodes;
+    ls.quantOnly = false;
     ls.sortHits = rs.sortHits;
     const size_t lanes = (size_t)ls.traceGrid * kTraceBlock;
     RBH_ALLOC(c, rs.spill, trace_spill_words(lanes) * sizeof(int));
@@ -622,12 +622,12 @@ int rbh_render(rbh_ctx c, const rbh_launch_params* lp) {
     const size_t NP = P * S;
     rc = prepare_accum(c, lp);
     if (rc) return rc;
-    if (rs.quantNodes && (rc = lbvh_quantise(c, c->stream)) != RBH_OK) return rc;
     Frame1 f{};
     fill_view(c, lp, f.sc);
     LaunchShape ls;
     rc = prepare_pass_state(c, NP, f, ls);
     if (rc) return rc;
+    ls.quantOnly = f.sc.nnodes4 > kMaxNodes4;
     f.maxP = (uint32_t)P;
     f.noDrop = (guided || (lp->flags & RBH_RENDER_NO_DROP)) ? 1u : 0u;
     f.camOrigin0 = lp->depthOfField ? 0u : 1u;
@@ -720,10 +720,6 @@ int rbh_render_batch(rbh_ctx owner, const rbh_ctx* scenes, const rbh_launch_para
                                               (unsigned long long)maxFilm);
     std::vector<SceneView> base(n);
     for (uint32_t s = 0; s < n; ++s) {
-        if (rs.quantNodes) {
-            const int rq = lbvh_quantise(scenes[s], owner->stream);
-            if (rq) return fail(owner, rq, "scene %u: %s", s, scenes[s]->err.c_str());
-        }
         fill_view(scenes[s], &lps[s], base[s]);
         // a scene may need fewer bounces than the pass runs; its paths end at its own caps
     }
@@ -772,6 +768,7 @@ int rbh_render_batch(rbh_ctx owner, const rbh_ctx* scenes, const rbh_launch_para
     LaunchShape ls;
     int rc = prepare_pass_state(owner, (size_t)passSlots, f, ls);
     if (rc) return rc;
+    for (const SceneView& v : base) ls.quantOnly = ls.quantOnly || v.nnodes4 > kMaxNodes4;
     f.noDrop = 0u;
     f.camOrigin0 = 1u;
     for (uint32_t s = 0; s < n; ++s) {
@@ -917,7 +914,7 @@ int rbh_autotune(rbh_ctx c, const rbh_launch_params* lp, uint32_t trialSpp, rbh_
         }
     }
     if (bestRate >= 0.0) {
-        // the 64-byte quantised nodes
+        // the nodes on an 11-bit grid
         rs.traceBlocksPerCU = b.traceBlocksPerCU;
         rs.shadeBlocksPerCU = b.shadeBlocksPerCU;
         rs.shadeWaves = b.shadeWaves ? b.shadeWaves : 1;

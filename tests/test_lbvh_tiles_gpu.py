@@ -5,7 +5,7 @@ against the binary tree's, after a build and after a refit."""
 import numpy as np
 import pytest
 
-from test_lbvh_gpu import _rays, _read_lbvh, _trace, _upload
+from test_lbvh_gpu import _brute, _rays, _read_lbvh, _trace, _upload
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,43 @@ def test_tiles_and_groups(ctx, n, spread):
         assert np.array_equal(a[:, 0], b[:, 0])
         q = _trace(ctx, rays, False, quant=True)
         assert np.array_equal(a[:, 0], q[:, 0])
+
+
+@pytest.mark.parametrize("which", ["axis-parallel", "far", "tiny", "huge"])
+def test_grid_nodes_at_the_ends_of_their_range(ctx, which):
+    # child boxes on the node's 11-bit grid only ever grow: the closest hit is
+    # the brute-force one for rays along box faces, origins far outside and
+    # scales far from one (the triangle test itself holds third powers)
+    rng = np.random.default_rng(7)
+    n = 3000
+    c = rng.integers(-6, 7, (n, 3)).astype(np.float64)
+    e = np.eye(3)[rng.permuted(np.tile([0, 1, 2], (n, 1)), axis=1)]   # two axis-aligned edges each
+    v = np.stack([c, c + e[:, 0], c + e[:, 1]], 1).reshape(-1, 3)
+    scale = {"tiny": 2.0 ** -30, "huge": 2.0 ** 30}.get(which, 1.0)
+    rays = _rays(rng, 4000, -7, 7)
+    if which == "axis-parallel":
+        d = np.zeros((4000, 3))
+        d[np.arange(4000), rng.integers(0, 3, 4000)] = rng.choice([-1.0, 1.0], 4000)
+        rays[:, 4:7] = d
+        rays[:, 0:3] = rng.integers(-28, 29, (4000, 3)) / 4.0
+        rays[2000:, 4:7] = np.where(rays[2000:, 4:7] == 0, np.float32(-0.0), rays[2000:, 4:7])
+    elif which == "far":
+        o = rays[:, 0:3] - 1e5 * rays[:, 4:7]
+        rays[:, 0:3] = o
+    rays[:, 0:3] *= np.float32(scale)
+    v = (v * scale).astype(np.float32)
+    idx = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    _upload(ctx, v, idx)
+    g, b = _trace(ctx, rays, False, quant=True), _brute(v, idx, rays, False)
+    hit = b[:, 1].view(np.uint32) != 0xFFFFFFFF
+    assert hit.sum() > 500
+    assert np.array_equal(g[:, 1].view(np.uint32) != 0xFFFFFFFF, hit)
+    # the same triangle test on both sides: a few ulp
+    np.testing.assert_allclose(g[hit, 0], b[hit, 0], rtol=1e-6)
+    if which != "axis-parallel":   # rays in a face pass the boxes of the other nodes by
+        f = _trace(ctx, rays, False)
+        assert np.array_equal(f[:, 0], g[:, 0])
+    # any hit: occluded exactly where there is a closest hit within the range
+    rays[:, 7] = np.where(hit, b[:, 0] * np.float32(1.001), np.float32(3e38))
+    a = _trace(ctx, rays, True, quant=True)
+    assert np.array_equal(a[:, 1].view(np.uint32) != 0xFFFFFFFF, hit)
