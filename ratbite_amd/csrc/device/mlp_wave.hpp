@@ -5,8 +5,8 @@
 // a layer loaded once for all its column tiles), outputs. Waves never wait
 // for each other; the LDS hand-over between lanes of one wave is ordered by
 // wavefront-scope fences. The arithmetic (bf16 activations, FP32
-// accumulation, bias added after the product, per-tile FP8 activation scale)
-// is that of the block-tiled forward pass in mlp.hpp.
+// accumulation, bias added after the product) is that of the training
+// kernel's forward pass.
 #pragma once
 #include <type_traits>
 
@@ -189,8 +189,8 @@ __device__ __forceinline__ WaveRec load_rec(const float* __restrict__ recs, uint
     return w;
 }
 
-// encodes the wave's 16 records into x0: the features of enc_feature, each
-// sin/cos pair from one sincospif; lane (r, g) writes pairs g, g + 4, ... of
+// encodes the wave's 16 records into x0: features 24 a + 2 k and + 1 are
+// sin and cos of 2^k pi position[a], each pair from one sincospif; lane (r, g) writes pairs g, g + 4, ... of
 // record r and features 72 + g, 76 + g, ...
 __device__ __forceinline__ void wave_encode(bf16* x0, const WaveRec& w, bool live) {
     const int lane = __lane_id(), r = lane & 15, g = lane >> 4;

@@ -55,9 +55,9 @@ struct GuideState {
     void* wf = nullptr;                // bf16 forward weights (kWfTotal)
     void* wt = nullptr;                // bf16 transposed weights (kWfTotal)
     void* bias = nullptr;              // float[kBiasPad]
-    void* partials = nullptr;          // float[blocks][kParams + kBiasPad]
+    void* partials = nullptr;          // float[blocks][kParams]
     size_t partialBlocks = 0;
-    void* scalars = nullptr;           // float[4]: weight sum, loss sum
+    void* scalars = nullptr;           // floats: loss and weight sums, then their partial sums per block
     void* records = nullptr;           // pending records of a collecting render (float[cap][24])
     void* trainRecs = nullptr;         // finished training records (float[cap][kRec])
     void* recCount = nullptr;          // uint32 counter
