@@ -24,6 +24,7 @@
 // back to the reference's binary search otherwise. FP64 mode carries the
 // prefix sums and the normalisation in double and rounds each CDF value once.
 #include "../context.hpp"
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -174,6 +175,60 @@ __device__ __forceinline__ void group_scan(T (&x)[V / WPR], T (&y)[V / WPR], T (
         x[k] += total; y[k] += total; z[k] += total; w[k] += total;
     }
     total = __shfl(col[V - 1] + total, 63);
+}
+
+// The value of the lane that a DPP control names, 0 where there is none or
+// its row is masked.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xF, false);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+// Inclusive prefixes of all NC chunks of a row in double precision, where no
+// order of the additions is prescribed: component prefixes, a DPP scan of
+// every register's 64 lanes, and the totals of the NC V registers of the row
+// exchanged once. `total` receives the row's sum. (The reference's order with
+// its cross-lane reads and two barriers a chunk: rows of 8192 texels 158 us
+// a 4096-row map, this way 123 us; the bytes alone 75 us.)
+template <int V, int WPR, int NC>
+__device__ __forceinline__ void row_scan_f64(double (&x)[NC][V / WPR], double (&y)[NC][V / WPR], double (&z)[NC][V / WPR],
+                                             double (&w)[NC][V / WPR], double& total, double* __restrict__ xtotal) {
+    constexpr int VW = V / WPR;
+    const int lane = __lane_id(), p = (int)(threadIdx.x >> 6);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+            y[c][k] += x[c][k];
+            z[c][k] += y[c][k];
+            w[c][k] += z[c][k];
+            double s = w[c][k];
+            s += dpp<0x111, 0xF>(s);   // row_shr 1, 2, 4, 8: prefixes of 16 lanes
+            s += dpp<0x112, 0xF>(s);
+            s += dpp<0x114, 0xF>(s);
+            s += dpp<0x118, 0xF>(s);
+            s += dpp<0x142, 0xA>(s);   // lane 15 of a row to the next, rows 1 and 3
+            s += dpp<0x143, 0xC>(s);   // lane 31 to rows 2 and 3
+            if (lane == 63) xtotal[c * V + p * VW + k] = s;
+            const double below = dpp<0x138, 0xF>(s);   // the lane below's prefix
+            x[c][k] += below; y[c][k] += below; z[c][k] += below; w[c][k] += below;
+        }
+    __syncthreads();
+    double run = 0.0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            // the registers of this wave take the sum of all before them
+#pragma unroll
+            for (int e = 0; e < VW; ++e)
+                if (k == p * VW + e) { x[c][e] += run; y[c][e] += run; z[c][e] += run; w[c][e] += run; }
+            run += xtotal[c * V + k];
+        }
+    total = run;
 }
 
 // Element (virtual lane) of register k of this wave in chunk c.
@@ -421,15 +476,19 @@ __device__ __forceinline__ void zero_marks(uint16_t* __restrict__ marks, int n) 
     for (int q = (int)threadIdx.x; 4 * q < n; q += 64 * WPR) z64[q] = make_uint2(0u, 0u);
 }
 
-// One workgroup of WPR waves per row: the row's power prefixes in
-// registers (chunks of the reference's B = 64 V lanes, running total between
-// chunks), the normalised CDF in the workgroup's LDS row, the row's inverted
-// indices from LDS, and the row's marginal term for the marginal kernel.
-// FP32 normalises the prefixes as it stores them when the row is one chunk,
-// otherwise keeps them in LDS and normalises them in place; FP64 scans the
-// row twice (the second time from L2) and rounds each normalised value to
-// float once.
-template <int V, int WPR, typename T>
+// One workgroup of WPR waves per row: the row's power prefixes in registers
+// (chunks of the reference's B = 64 V lanes, running total between chunks),
+// the normalised CDF in the workgroup's LDS row, the row's inverted indices
+// from LDS, and the row's marginal term for the marginal kernel.
+// NC > 0: the row's NC chunks stay in registers from the load to the
+// normalisation (rows of up to 2 B lanes; four chunks spill). All loads are issued before the
+// first scan, and the scan's exchange rows lie in the LDS that the CDF takes
+// afterwards, which leaves room for a third workgroup per CU at 8192 texels:
+// 8192x4096 in FP64 264 -> 158 us.
+// NC = 0 (wider rows): FP32 keeps the prefixes in LDS and normalises them in
+// place; FP64 scans the row twice (the second time from L2) and rounds each
+// normalised value to float once.
+template <int V, int WPR, int NC, typename T>
 __global__ __launch_bounds__(64 * WPR) void k_envmap_rows(const float* __restrict__ texels, int w, int h, int channels,
                                                            uint16_t* __restrict__ cond, T* __restrict__ rowTotals) {
     constexpr int VW = V / WPR;
@@ -440,30 +499,42 @@ __global__ __launch_bounds__(64 * WPR) void k_envmap_rows(const float* __restric
     __shared__ uint32_t segMax[WPR];
     float* cdf = lds;
     uint16_t* marks = use_marks(w) ? reinterpret_cast<uint16_t*>(cdf + w) : nullptr;
-    T* xcol = reinterpret_cast<T*>(lds + wave_lds_floats(w));
+    T* xcol = reinterpret_cast<T*>(NC > 0 ? lds : lds + wave_lds_floats(w));
     T* xghost = xcol + V * 64;
     const int row = blockIdx.x;
     const int numEl = w >> 2;
     const int nChunks = (numEl + B - 1) / B;
     const float* rowp = texels + (size_t)row * w * channels;
-    zero_marks<WPR>(marks, w);
-    if (threadIdx.x == 0) badFlag = 0;
-    // (the scan's barriers order these before the inversion)
 
     T total = (T)0;
-    for (int c = 0; c < nChunks; ++c) {
-        T x[VW], y[VW], z[VW], q[VW];
-        load_part<V, WPR, T>(rowp, numEl, c, channels, x, y, z, q);
-        group_scan<V, WPR, T>(x, y, z, q, total, xcol, xghost);
+    if constexpr (NC > 0) {
+        T x[NC][VW], y[NC][VW], z[NC][VW], q[NC][VW];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) load_part<V, WPR, T>(rowp, numEl, c, channels, x[c], y[c], z[c], q[c]);
+        if (threadIdx.x == 0) badFlag = 0;
         if constexpr (kF32) {
-            // cdf.cu:380-392: a one-chunk row is normalised as it is stored
-            const T norm = total != (T)0 ? (T)1 / total : (T)0;
-            store_part_lds<V, WPR, T>(cdf, numEl, c, x, y, z, q, nChunks == 1, norm);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) group_scan<V, WPR, T>(x[c], y[c], z[c], q[c], total, xcol, xghost);
+        } else {
+            row_scan_f64<V, WPR, NC>(x, y, z, q, total, xcol);
         }
-    }
-    const T norm = total != (T)0 ? (T)1 / total : (T)0;
-    if constexpr (kF32) {
-        if (nChunks > 1) {
+        const T norm = total != (T)0 ? (T)1 / total : (T)0;   // cdf.cu:380-392
+        __syncthreads();   // the exchange rows become the CDF and the marks
+        zero_marks<WPR>(marks, w);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) store_part_lds<V, WPR, T>(cdf, numEl, c, x[c], y[c], z[c], q[c], true, norm);
+    } else {
+        zero_marks<WPR>(marks, w);
+        if (threadIdx.x == 0) badFlag = 0;
+        // (the scan's barriers order these before the inversion)
+        for (int c = 0; c < nChunks; ++c) {
+            T x[VW], y[VW], z[VW], q[VW];
+            load_part<V, WPR, T>(rowp, numEl, c, channels, x, y, z, q);
+            group_scan<V, WPR, T>(x, y, z, q, total, xcol, xghost);
+            if constexpr (kF32) store_part_lds<V, WPR, T>(cdf, numEl, c, x, y, z, q, false, (T)1);
+        }
+        const T norm = total != (T)0 ? (T)1 / total : (T)0;
+        if constexpr (kF32) {
             // in place, each lane rescaling what it wrote
             for (int c = 0; c < nChunks; ++c)
 #pragma unroll
@@ -476,14 +547,14 @@ __global__ __launch_bounds__(64 * WPR) void k_envmap_rows(const float* __restric
                         *e = v;
                     }
                 }
-        }
-    } else {
-        T t2 = (T)0;
-        for (int c = 0; c < nChunks; ++c) {
-            T x[VW], y[VW], z[VW], q[VW];
-            load_part<V, WPR, T>(rowp, numEl, c, channels, x, y, z, q);
-            group_scan<V, WPR, T>(x, y, z, q, t2, xcol, xghost);
-            store_part_lds<V, WPR, T>(cdf, numEl, c, x, y, z, q, true, norm);
+        } else {
+            T t2 = (T)0;
+            for (int c = 0; c < nChunks; ++c) {
+                T x[VW], y[VW], z[VW], q[VW];
+                load_part<V, WPR, T>(rowp, numEl, c, channels, x, y, z, q);
+                group_scan<V, WPR, T>(x, y, z, q, t2, xcol, xghost);
+                store_part_lds<V, WPR, T>(cdf, numEl, c, x, y, z, q, true, norm);
+            }
         }
     }
     // the row's marginal term: its total times the row weight (cdf.cu:112-132),
@@ -592,18 +663,36 @@ hipError_t set_lds(K fn, size_t lds) {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
+template <int V, int WPR, int NC, typename T>
+hipError_t launch_rows(hipStream_t s, const float* texels, int w, int h, int ch, uint16_t* cond, T* rowTotals) {
+    // NC > 0: the exchange rows share the CDF's LDS
+    const size_t exchange = (size_t)(V + WPR) * 64 * sizeof(T);
+    const size_t lds = NC > 0 ? std::max(wave_lds_floats(w) * sizeof(float), exchange) : cdf_lds_bytes<T>(w, V, WPR);
+    auto rows = k_envmap_rows<V, WPR, NC, T>;
+    const hipError_t e = set_lds(rows, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(rows, dim3(h), dim3(64 * WPR), lds, s, texels, w, h, ch, cond, rowTotals);
+    return hipGetLastError();
+}
+
 template <int V, int WPR, typename T>
 hipError_t launch_cdf_v(hipStream_t s, const float* texels, int w, int h, int ch, uint16_t* cond, uint16_t* marg,
                         float* cdfY, void* rowTotals, void* integral, double* normIntegral) {
-    const size_t ldsRows = cdf_lds_bytes<T>(w, V, WPR), ldsMarg = cdf_lds_bytes<T>(h, V, WPR);
-    auto rows = k_envmap_rows<V, WPR, T>;
+    const size_t ldsMarg = cdf_lds_bytes<T>(h, V, WPR);
     auto margK = k_envmap_marginal<V, WPR, T>;
-    hipError_t e = set_lds(rows, ldsRows);
-    if (e == hipSuccess) e = set_lds(margK, ldsMarg);
+    hipError_t e = set_lds(margK, ldsMarg);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(rows, dim3(h), dim3(64 * WPR), ldsRows, s, texels, w, h, ch, cond, static_cast<T*>(rowTotals));
-    hipLaunchKernelGGL(margK, dim3(1), dim3(64 * WPR), ldsMarg, s, w, h, marg, cdfY, static_cast<T*>(rowTotals),
-                       static_cast<T*>(integral), normIntegral);
+    // rows of more than one chunk have the largest block (V = 16)
+    T* rt = static_cast<T*>(rowTotals);
+    const int chunks = ((w >> 2) + 64 * V - 1) / (64 * V);
+    if (chunks <= 1) e = launch_rows<V, WPR, 1, T>(s, texels, w, h, ch, cond, rt);
+    else if constexpr (V == 16) {
+        if (chunks == 2) e = launch_rows<V, WPR, 2, T>(s, texels, w, h, ch, cond, rt);
+        else e = launch_rows<V, WPR, 0, T>(s, texels, w, h, ch, cond, rt);
+    }
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(margK, dim3(1), dim3(64 * WPR), ldsMarg, s, w, h, marg, cdfY, rt, static_cast<T*>(integral),
+                       normIntegral);
     return hipGetLastError();
 }
 
