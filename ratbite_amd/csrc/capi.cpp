@@ -134,7 +134,7 @@ int rbh_upload_textures(rbh_ctx c, const rbh_texture_desc* descs, uint32_t n, co
     RBH_ALLOC(c, c->textures, (size_t)(n ? n : 1) * sizeof(TextureDesc));
     RBH_ALLOC(c, c->texels, blobBytes ? blobBytes : 16);
     if (n) RBH_HIP(c, hipMemcpyAsync(c->textures.p, descs, (size_t)n * sizeof(TextureDesc), hipMemcpyHostToDevice, c->stream));
-    if (blobBytes) RBH_HIP(c, hipMemcpyAsync(c->texels.p, blob, blobBytes, hipMemcpyHostToDevice, c->stream));
+    if (blobBytes) RBH_HIP(c, copy_in(c, c->texels.p, blob, blobBytes));
     RBH_ALLOC(c, c->srgbLut, 256 * sizeof(float));
     RBH_HIP(c, rbh::srgb_lut_fill(c));
     RBH_HIP(c, hipStreamSynchronize(c->stream));
@@ -217,11 +217,11 @@ int rbh_upload_geometry_ex(rbh_ctx c, const float* verts, uint32_t nverts, const
     RBH_ALLOC(c, g.attribs, attribBytes ? attribBytes : 16);
     RBH_ALLOC(c, g.triMaterial, (size_t)ntris * 4);
     RBH_ALLOC(c, g.triLight, (size_t)ntris * 4);
-    RBH_HIP(c, hipMemcpyAsync(g.verts.p, verts, (size_t)nverts * 12, hipMemcpyHostToDevice, c->stream));
-    RBH_HIP(c, hipMemcpyAsync(g.indices.p, indices, (size_t)ntris * 12, hipMemcpyHostToDevice, c->stream));
-    if (attribBytes) RBH_HIP(c, hipMemcpyAsync(g.attribs.p, attribs, attribBytes, hipMemcpyHostToDevice, c->stream));
-    RBH_HIP(c, hipMemcpyAsync(g.triMaterial.p, triMaterial, (size_t)ntris * 4, hipMemcpyHostToDevice, c->stream));
-    RBH_HIP(c, hipMemcpyAsync(g.triLight.p, triLight, (size_t)ntris * 4, hipMemcpyHostToDevice, c->stream));
+    RBH_HIP(c, copy_in(c, g.verts.p, verts, (size_t)nverts * 12));
+    RBH_HIP(c, copy_in(c, g.indices.p, indices, (size_t)ntris * 12));
+    if (attribBytes) RBH_HIP(c, copy_in(c, g.attribs.p, attribs, attribBytes));
+    RBH_HIP(c, copy_in(c, g.triMaterial.p, triMaterial, (size_t)ntris * 4));
+    RBH_HIP(c, copy_in(c, g.triLight.p, triLight, (size_t)ntris * 4));
     RBH_HIP(c, hipStreamSynchronize(c->stream));
     g.nverts = nverts;
     g.ntris = ntris;
@@ -280,7 +280,7 @@ int rbh_envmap_build(rbh_ctx c, const float* texels, int w, int h, int ch, uint3
     RBH_ALLOC(c, e.cdfY, (size_t)h * sizeof(float));
     RBH_ALLOC(c, e.integralDev, envmap_scratch_bytes(h));
     e.width = w; e.height = h; e.channels = ch;
-    RBH_HIP(c, hipMemcpyAsync(e.texels.p, texels, (size_t)w * h * ch * sizeof(float), hipMemcpyHostToDevice, c->stream));
+    RBH_HIP(c, copy_in(c, e.texels.p, texels, (size_t)w * h * ch * sizeof(float)));
     int r = envmap_run(c, flags);
     if (r) return r;
     return envmap_finish(c, flags);
@@ -320,7 +320,7 @@ int rbh_envmap_read(rbh_ctx c, uint16_t* cond, uint16_t* marg, float* cdfY, doub
     if (!c->env.enabled) return fail(c, RBH_ERR_STATE, "no environment map built");
     const EnvMap& e = c->env;
     RBH_HIP(c, hipStreamSynchronize(c->stream));
-    if (cond) RBH_HIP(c, hipMemcpy(cond, e.cond.p, (size_t)e.width * e.height * 2, hipMemcpyDeviceToHost));
+    if (cond) RBH_HIP(c, copy_out(c, cond, e.cond.p, (size_t)e.width * e.height * 2));
     if (marg) RBH_HIP(c, hipMemcpy(marg, e.marg.p, (size_t)e.height * 2, hipMemcpyDeviceToHost));
     if (cdfY) RBH_HIP(c, hipMemcpy(cdfY, e.cdfY.p, (size_t)e.height * 4, hipMemcpyDeviceToHost));
     if (integral) *integral = e.integral;

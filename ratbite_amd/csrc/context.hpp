@@ -5,12 +5,16 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdarg>
+#include <memory>
 #include <string>
 #include <vector>
 #include "../../include/ratbite_hip.h"
 #include "device/types.hpp"
+#include "host_copy.hpp"
 
 namespace rbh {
+
+class CopyPool;   // host_copy.cpp
 
 // Owning device allocation.
 struct DevBuf {
@@ -183,6 +187,9 @@ struct rbh_context {
     rbh::RenderState rs;
     rbh_stats stats{};
     void* guide = nullptr;    // guiding state (guide.hip)
+    rbh::DevBuf guideRecords, guideOutputs;   // a caller's records on the device, and their outputs
+    std::shared_ptr<rbh::CopyPool> copyPool;   // the device's threads for large host copies, from the first one on
+    bool copyPoolFailed = false;
 };
 
 namespace rbh {

@@ -755,21 +755,22 @@ int rbh_guide_get_params(rbh_ctx c, float* params, uint32_t n) {
     return RBH_OK;
 }
 
-static int stage_records(rbh_ctx c, const float* recs, uint32_t n, DevBuf& buf) {
+static int stage_records(rbh_ctx c, const float* recs, uint32_t n) {
+    DevBuf& buf = c->guideRecords;
     RBH_ALLOC(c, buf, (size_t)std::max<uint32_t>(n, 1) * kRec * 4);
-    RBH_HIP(c, hipMemcpyAsync(buf.p, recs, (size_t)n * kRec * 4, hipMemcpyHostToDevice, c->stream));
+    RBH_HIP(c, copy_in(c, buf.p, recs, (size_t)n * kRec * 4));
     return RBH_OK;
 }
 
 int rbh_guide_gradient(rbh_ctx c, const float* recs, uint32_t n, float* grad, float* loss) {
     if (!c || !recs || !grad || n == 0) return RBH_ERR_INVALID;
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
-    DevBuf d, gbuf;
-    int rc = stage_records(c, recs, n, d);
+    DevBuf gbuf;
+    int rc = stage_records(c, recs, n);
     if (rc) return rc;
     RBH_ALLOC(c, gbuf, kParams * 4);
     float l = 0.0f;
-    rc = run_train(c, d.as<float>(), n, 1, gbuf.as<float>(), &l);
+    rc = run_train(c, c->guideRecords.as<float>(), n, 1, gbuf.as<float>(), &l);
     if (rc) return rc;
     RBH_HIP(c, hipMemcpy(grad, gbuf.p, kParams * 4, hipMemcpyDeviceToHost));
     if (loss) *loss = l;
@@ -779,11 +780,10 @@ int rbh_guide_gradient(rbh_ctx c, const float* recs, uint32_t n, float* grad, fl
 int rbh_guide_train(rbh_ctx c, const float* recs, uint32_t n, uint32_t batch, uint32_t steps, float* lastLoss) {
     if (!c || !recs || n == 0 || batch == 0) return RBH_ERR_INVALID;
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
-    DevBuf d;
-    int rc = stage_records(c, recs, n, d);
+    int rc = stage_records(c, recs, n);
     if (rc) return rc;
     float l = 0.0f;
-    rc = run_steps(c, d.as<float>(), n, batch, steps, &l);
+    rc = run_steps(c, c->guideRecords.as<float>(), n, batch, steps, &l);
     if (rc) return rc;
     if (lastLoss) *lastLoss = l;
     return RBH_OK;
@@ -805,7 +805,7 @@ int rbh_guide_records(rbh_ctx c, float* out, uint32_t max, uint32_t* n) {
     int rc = collected(c, &k);
     if (rc) return rc;
     *n = k;
-    if (out && max) RBH_HIP(c, hipMemcpy(out, gs(c).trainRecs, (size_t)std::min(k, max) * kRec * 4, hipMemcpyDeviceToHost));
+    if (out && max) RBH_HIP(c, copy_out(c, out, gs(c).trainRecs, (size_t)std::min(k, max) * kRec * 4));
     return RBH_OK;
 }
 
@@ -869,9 +869,9 @@ static int infer(rbh_ctx c, const float* recs, uint32_t n, float* out, bool fp8)
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
     if (n == 0) return RBH_OK;
     GuideState& g = gs(c);
-    DevBuf d, o;
-    int rc = stage_records(c, recs, n, d);
+    int rc = stage_records(c, recs, n);
     if (rc) return rc;
+    DevBuf &d = c->guideRecords, &o = c->guideOutputs;
     RBH_ALLOC(c, o, (size_t)n * kOut * 4);
     // four waves of 16 records per block
     const int blocks = (int)std::min<size_t>((size_t)train_blocks(c) * 2, (n + 4 * kRows - 1) / (4 * kRows));
@@ -882,8 +882,7 @@ static int infer(rbh_ctx c, const float* recs, uint32_t n, float* out, bool fp8)
         hipLaunchKernelGGL((k_guide_infer<false>), dim3(blocks), dim3(256), 0, c->stream, d.as<float>(), n,
                            dptr<bf16>(g.wf), nullptr, dptr<float>(g.fp8s), dptr<float>(g.bias), o.as<float>());
     RBH_HIP(c, hipGetLastError());
-    RBH_HIP(c, hipStreamSynchronize(c->stream));
-    RBH_HIP(c, hipMemcpy(out, o.p, (size_t)n * kOut * 4, hipMemcpyDeviceToHost));
+    RBH_HIP(c, copy_out(c, out, o.p, (size_t)n * kOut * 4));
     return RBH_OK;
 }
 

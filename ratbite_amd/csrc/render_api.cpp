@@ -88,8 +88,7 @@ int rbh_update_vertices(rbh_ctx c, uint32_t first, uint32_t count, const float* 
     if ((uint64_t)first + count > g.nverts)
         return fail(c, RBH_ERR_RANGE, "vertices %u..%u of %u", first, first + count, g.nverts);
     if (!count) return RBH_OK;
-    RBH_HIP(c, hipMemcpyAsync(g.verts.as<char>() + (size_t)first * 12, verts, (size_t)count * 12,
-                              hipMemcpyHostToDevice, c->stream));
+    RBH_HIP(c, copy_in(c, g.verts.as<char>() + (size_t)first * 12, verts, (size_t)count * 12));
     RBH_HIP(c, hipStreamSynchronize(c->stream));
     c->accel.stale = true;
     return RBH_OK;
@@ -1057,15 +1056,14 @@ int rbh_set_path_slots(rbh_ctx c, uint64_t slots) {
 int rbh_read_accum(rbh_ctx c, double* rgbw) {
     if (!c || !rgbw) return RBH_ERR_INVALID;
     if (!c->rs.accum.p) return fail(c, RBH_ERR_STATE, "nothing rendered");
-    RBH_HIP(c, hipStreamSynchronize(c->stream));
-    RBH_HIP(c, hipMemcpy(rgbw, c->rs.accum.p, (size_t)c->rs.width * c->rs.height * 32, hipMemcpyDeviceToHost));
+    RBH_HIP(c, copy_out(c, rgbw, c->rs.accum.p, (size_t)c->rs.width * c->rs.height * 32));
     return RBH_OK;
 }
 
 int rbh_write_accum(rbh_ctx c, const double* rgbw, uint32_t w, uint32_t h) {
     if (!c || !rgbw || w == 0 || h == 0) return RBH_ERR_INVALID;
     RBH_ALLOC(c, c->rs.accum, (size_t)w * h * 32);
-    RBH_HIP(c, hipMemcpyAsync(c->rs.accum.p, rgbw, (size_t)w * h * 32, hipMemcpyHostToDevice, c->stream));
+    RBH_HIP(c, copy_in(c, c->rs.accum.p, rgbw, (size_t)w * h * 32));
     RBH_HIP(c, hipStreamSynchronize(c->stream));
     c->rs.width = w;
     c->rs.height = h;
@@ -1078,8 +1076,7 @@ int rbh_resolve(rbh_ctx c, const float* colorspace, float exposureScale, uint8_t
     const size_t n = (size_t)c->rs.width * c->rs.height;
     RBH_ALLOC(c, c->rs.image, n * 4);
     RBH_HIP(c, resolve_launch(c, colorspace, exposureScale, c->rs.image.p));
-    RBH_HIP(c, hipMemcpyAsync(rgba8, c->rs.image.p, n * 4, hipMemcpyDeviceToHost, c->stream));
-    RBH_HIP(c, hipStreamSynchronize(c->stream));
+    RBH_HIP(c, copy_out(c, rgba8, c->rs.image.p, n * 4));
     return RBH_OK;
 }
 
