@@ -484,13 +484,20 @@ __global__ __launch_bounds__(kShadeBlock, WAVES) void k_shade(Frame1 f, uint32_t
 // the separate kernels (0.68 ms with one lane per path), 640x360 over 1M
 // triangles with a refit 3.9 against 5.3 ms. bounce: the bounce the queue
 // belongs to (0: every slot starts with its camera ray).
-// kTailPaths: 4096 waves, two resident rounds of the kernel's two waves per
-// SIMD. Measured at 16k / 64k / 128k / 256k paths: 256x256x16 Cornell 3.68 /
+// kTailPaths: 4096 waves. Measured at 16k / 64k / 128k / 256k paths: 256x256x16 Cornell 3.68 /
 // 3.61 / 3.72 / 4.10 ms, feature scene 333x187x8 2.40 / 2.36 / 2.53 / 2.92 ms,
 // 1080p x 64 spp of 4.1M triangles 114.3 / 114.1 / 116.3 / 122.3 ms.
 constexpr uint32_t kTailPaths = 65536u;
-template <bool BATCH>
-__global__ __launch_bounds__(kPathBlock) void k_paths(Frame1 f, uint32_t bounce, uint32_t depthMax) {
+// Waves per SIMD: a tail is up to 4096 waves, two rounds at two waves per SIMD
+// (227 registers) and better off with a few spills and three: feature scene
+// 333x187x8 2.27 -> 2.17 ms, edit of 1M triangles with a 640x360 preview 2.85 ->
+// 2.62 ms (four waves: 2.24 / 2.85 ms). Up to kFewPaths are resident at once
+// either way, and the registers shorten their chain: 64x64 preview 0.485 against
+// 0.502 ms.
+constexpr int kTailWaves = 3;
+constexpr uint32_t kFewPaths = 32768u;
+template <bool BATCH, int WAVES>
+__global__ __launch_bounds__(kPathBlock, WAVES) void k_paths(Frame1 f, uint32_t bounce, uint32_t depthMax) {
     __shared__ int stack[kQuadStackLds * kQuadRays];
     const uint32_t t = (blockIdx.x * kPathBlock + threadIdx.x) >> 2;
     const TravStack<kQuadStackLds> st{stack + (threadIdx.x >> 2), kQuadRays, f.spill + t, f.spillStride};
@@ -654,13 +661,16 @@ static hipError_t launch_pass_t(rbh_ctx c, Frame1 f, uint32_t depthMax, const La
     const dim3 pathGrid(std::min<uint32_t>((std::min(std::max(f.tail, 1u), f.NP) + kQuadRays - 1) / kQuadRays,
                                            (uint32_t)ls.traceGrid * kTraceBlock / kQuadRays));
     const bool allPaths = f.NP <= f.tail;
-    if (allPaths) hipLaunchKernelGGL((k_paths<BATCH>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
+    if (allPaths && f.NP <= kFewPaths)
+        hipLaunchKernelGGL((k_paths<BATCH, 2>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
+    else if (allPaths)
+        hipLaunchKernelGGL((k_paths<BATCH, kTailWaves>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
     for (uint32_t b = 0; b < depthMax && !allPaths; ++b) {
         const uint32_t qsel = b & 1u;
         f.bounce = b;
         f.counters = counters + b * CNT_COUNT;
         if (f.tail && b > 0)
-            hipLaunchKernelGGL((k_paths<BATCH>), pathGrid, dim3(kPathBlock), 0, c->stream, f, b, depthMax);
+            hipLaunchKernelGGL((k_paths<BATCH, kTailWaves>), pathGrid, dim3(kPathBlock), 0, c->stream, f, b, depthMax);
         RBH_TIMED(KernelTimer::TRACE, launch_trace<BATCH>(c, f, qsel, ls));
         RBH_TIMED(KernelTimer::SHADE,
                   hipLaunchKernelGGL(k_miss<BATCH>, dim3(ls.shadeGrid), dim3(256), 0, c->stream, f));

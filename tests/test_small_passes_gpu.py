@@ -77,3 +77,14 @@ def test_pass_size_leaves_the_image_bits(ctx, make, no_drop):
     assert np.array_equal(big, r.accum())
     assert [a[k] for k in ("closestRays", "shadowRays", "pathVertices")] == \
         [b[k] for k in ("closestRays", "shadowRays", "pathVertices")]
+
+
+@pytest.mark.parametrize("width,height", [(256, 128), (257, 128), (256, 256), (257, 256)])
+def test_pass_sizes_where_the_register_budget_changes(ctx, width, height):
+    # 32768 paths are the last that run with the larger register budget, 65536
+    # the last that are one kernel from the start
+    r = Renderer(scenes.features(width=width, height=height), ctx=ctx)
+    r.render(spp=1, offset=0)
+    a = r.accum()
+    r.render(spp=1, offset=0, flags=L.RBH_RENDER_TIMING)
+    assert np.array_equal(a, r.accum())
