@@ -127,13 +127,12 @@ private:
         const auto size = [this](size_t off) { return std::min(chunk_, bytes_ - off); };
         if (toHost_) {
             size_t off[2] = {claim(), 0};
-            if (off[0] >= bytes_ || !fetch(k, 0, off[0], size(off[0]))) return;
-            for (int s = 0;; s ^= 1) {
+            bool more = off[0] < bytes_ && fetch(k, 0, off[0], size(off[0]));
+            for (int s = 0; more; s ^= 1) {
                 off[s ^ 1] = claim();
-                const bool more = off[s ^ 1] < bytes_ && fetch(k, s ^ 1, off[s ^ 1], size(off[s ^ 1]));
+                more = off[s ^ 1] < bytes_ && fetch(k, s ^ 1, off[s ^ 1], size(off[s ^ 1]));
                 if (!ok(hipEventSynchronize(event_[k][s]))) break;
                 std::memcpy(dst_ + off[s], slot(k, s), size(off[s]));
-                if (!more) break;
             }
         } else {
             bool used[2] = {false, false};
