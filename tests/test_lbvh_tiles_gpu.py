@@ -5,6 +5,7 @@ against the binary tree's, after a build and after a refit."""
 import numpy as np
 import pytest
 
+from ratbite_amd import _lib as L
 from test_lbvh_gpu import _brute, _rays, _read_lbvh, _trace, _upload
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +104,61 @@ def test_grid_nodes_at_the_ends_of_their_range(ctx, which):
     rays[:, 7] = np.where(hit, b[:, 0] * np.float32(1.001), np.float32(3e38))
     a = _trace(ctx, rays, True, quant=True)
     assert np.array_equal(a[:, 1].view(np.uint32) != 0xFFFFFFFF, hit)
+
+
+def _with_bad_triangles(n, bad, kind, seed):
+    """Valid triangles around the origin and then bad ones, whose x is not
+    finite (or spans more than a float holds) and whose y and z are near 100."""
+    rng = np.random.default_rng(seed)
+    v = (rng.uniform(-5, 5, (n, 1, 3)) + rng.normal(scale=0.3, size=(n, 3, 3))).astype(np.float32)
+    b = (100.0 + rng.random((bad, 3, 3))).astype(np.float32)
+    if kind == "nan":
+        b[..., 0] = np.nan
+    elif kind == "infinity":
+        b[..., 0] = np.inf
+    elif kind == "infinite-flat":
+        b[:, 0, 0], b[:, 1, 0], b[..., 1] = -np.inf, np.inf, 100.0
+    else:
+        b[:, 0, 0], b[:, 1, 0], b[..., 1] = -3e38, 3e38, 100.0
+    return np.concatenate([v, b]).reshape(-1, 3)
+
+
+def _rays_past(rng, n):
+    """Rays that stay clear of the bad triangles' y and z."""
+    r = _rays(rng, n, -6, 6)
+    lo, hi = (98.0 - r[:, 1:3]) / r[:, 5:7], (103.0 - r[:, 1:3]) / r[:, 5:7]
+    near, far = np.minimum(lo, hi).max(axis=1), np.maximum(lo, hi).min(axis=1)
+    return np.ascontiguousarray(r[(near > far) | (far < 0)])
+
+
+# the walks rbh_test_trace has (its mode bits) over full boxes
+FULL_WALKS = {"four-wide": 0, "binary": 4, "four lanes": 16}
+
+
+@pytest.mark.parametrize("kind", ["nan", "infinity", "infinite-flat", "overflow"])
+@pytest.mark.parametrize("n,bad", [(1, 2), (3, 61), (200, 40), (4000, 3000), (40000, 30000)])
+def test_vertices_that_are_not_finite(ctx, n, bad, kind):
+    # the other triangles are hit as if they were alone, after a build and
+    # after a refit
+    v = _with_bad_triangles(n, bad, kind, n + bad)
+    idx = np.arange(len(v), dtype=np.uint32).reshape(-1, 3)
+    rays = _rays_past(np.random.default_rng(11), 2000)
+    for refit in (False, True):
+        if refit:
+            v = np.roll(v.reshape(-1, 3, 3), 1, axis=1).reshape(-1, 3) + np.float32([0.0, 0.125, 0.0])
+            ctx.update_vertices(0, v)
+            ctx.refit_accel()
+        else:
+            _upload(ctx, v, idx)
+        b = _brute(v[:3 * n], idx[:n], rays, False)
+        hit = b[:, 1].view(np.uint32) != 0xFFFFFFFF
+        for name, mode in FULL_WALKS.items():
+            g = _trace_mode(ctx, rays, mode)
+            assert np.array_equal(g[:, 1].view(np.uint32) != 0xFFFFFFFF, hit), name
+            np.testing.assert_allclose(g[hit, 0], b[hit, 0], rtol=1e-5, atol=1e-5, err_msg=name)
+
+
+def _trace_mode(ctx, rays, mode):
+    hits = np.zeros((len(rays), 4), np.float32)
+    ctx.check(L.lib().rbh_test_trace(ctx.h, L.ptr(rays), L.ptr(hits), len(rays), mode))
+    return hits
