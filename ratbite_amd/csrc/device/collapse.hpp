@@ -43,10 +43,26 @@ __device__ __forceinline__ float half_area(const Box& b) {
     return x * y + y * z + z * x;
 }
 
+// A plane on the grid, rounded outwards (towards -inf for the lower ones). An
+// infinite one stays infinite (half floats have both), and a box without a
+// position on the axis (all vertices NaN) is open to that side.
+template <bool UPPER>
+__device__ __forceinline__ uint16_t grid_plane(float p, float o, int e) {
+    const float outside = UPPER ? INFINITY : -INFINITY;
+    float q = p == p ? p : outside;
+    if (fabsf(p) < INFINITY) {
+        const double x = ldexp((double)p - (double)o, -e);
+        q = (float)(UPPER ? ceil(x) : floor(x));
+    }
+    return __builtin_bit_cast(uint16_t, (_Float16)q);
+}
+
 // The 11-bit form of a four-wide node whose inner children come first. Grid
 // steps are powers of two and the arithmetic is in double precision, where a
 // difference of two floats divided by one is exact (or rounded by 2^-53, far
-// below the traversal's margin), so floor and ceil give planes outside.
+// below the traversal's margin), so floor and ceil give planes outside. The
+// grid spans the finite planes: beside an infinite vertex the other boxes
+// keep their resolution.
 __device__ __forceinline__ Bvh4HNode grid_node(const Bvh4Node& nd) {
     Bvh4HNode q;
     uint32_t tris = 0u, inner = 0u;
@@ -58,8 +74,14 @@ __device__ __forceinline__ Bvh4HNode grid_node(const Bvh4Node& nd) {
     }
     q.meta = tris << 24 | inner << 28;
     auto axis = [&](int a, const float (&lo)[4], const float (&hi)[4]) {
-        // empty boxes are (+inf, -inf)
-        const float o = fminf(fminf(lo[0], lo[1]), fminf(lo[2], lo[3])), top = fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3]));
+        float o = INFINITY, top = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {   // (empty boxes are (+inf, -inf))
+            const bool l = fabsf(lo[k]) < INFINITY, h = fabsf(hi[k]) < INFINITY;
+            o = fminf(o, fminf(l ? lo[k] : INFINITY, h ? hi[k] : INFINITY));
+            top = fmaxf(top, fmaxf(l ? lo[k] : -INFINITY, h ? hi[k] : -INFINITY));
+        }
+        if (o > top) o = top = 0.0f;   // none
         int e = 0;
         (void)frexp(((double)top - (double)o) / (double)kGridMax, &e);   // extent / 2047 < 2^e
         e = min(max(e, -126), 127);
@@ -67,9 +89,8 @@ __device__ __forceinline__ Bvh4HNode grid_node(const Bvh4Node& nd) {
         q.meta |= ((uint32_t)e & 0xFFu) << (8 * a);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const double l = floor(ldexp((double)lo[k] - (double)o, -e)), h = ceil(ldexp((double)hi[k] - (double)o, -e));
-            q.row[a][0][k] = __builtin_bit_cast(uint16_t, (_Float16)(float)l);
-            q.row[a][1][k] = __builtin_bit_cast(uint16_t, (_Float16)(float)h);
+            q.row[a][0][k] = grid_plane<false>(lo[k], o, e);
+            q.row[a][1][k] = grid_plane<true>(hi[k], o, e);
         }
     };
     axis(0, nd.lox, nd.hix);

@@ -101,3 +101,31 @@ def test_indices(lib, kind, n):
         # a node is short of children only if none of them could be opened
         short = (child == EMPTY).any(axis=1)
         assert not (child[short] >= 0).any()
+
+
+@pytest.mark.parametrize("kind", ["finite", "all-nan", "some-nan", "nan-axis", "infinite-flat", "overflow-flat", "one-infinity"])
+def test_grid_boxes_hold_the_full_ones(lib, kind):
+    # the 11-bit planes lie outside the full ones, the node's corner is finite
+    # and a box without a position on an axis is open there
+    for n in (2, 5, 64, 300):
+        rng = np.random.default_rng(n)
+        n4, n4h, writes, _ = collapse(lib, binary_tree(triangles(kind, n, rng), rng))
+        n4, n4h = n4[writes == 1], n4h[writes == 1]
+        assert np.isfinite(n4h["o"]).all()
+        full = n4["child"] != EMPTY
+        for a, (lo, hi) in enumerate((("lox", "hix"), ("loy", "hiy"), ("loz", "hiz"))):
+            e = ((n4h["meta"] >> np.uint32(8 * a)) & np.uint32(0xFF)).astype(np.int8).astype(np.float64)
+            with np.errstate(invalid="ignore"):
+                plane = n4h["o"][:, a, None, None].astype(np.float64) + \
+                    n4h["row"][:, a].astype(np.float64) * np.exp2(e)[:, None, None]
+            below, above = plane[:, 0][full], plane[:, 1][full]
+            l, h = n4[lo][full].astype(np.float64), n4[hi][full].astype(np.float64)
+            none = np.isnan(l)
+            assert np.array_equal(none, np.isnan(h))
+            assert np.all(below[none] == -np.inf) and np.all(above[none] == np.inf)
+            assert np.all(below[~none] <= l[~none]) and np.all(above[~none] >= h[~none])
+            # and within one step of them where they are finite
+            step = np.broadcast_to(np.exp2(e)[:, None], full.shape)[full]
+            for p, q in ((below, l), (above, h)):
+                f = np.isfinite(q)
+                assert np.all(np.abs(p[f] - q[f]) <= step[f])

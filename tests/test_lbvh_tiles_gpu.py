@@ -131,8 +131,8 @@ def _rays_past(rng, n):
     return np.ascontiguousarray(r[(near > far) | (far < 0)])
 
 
-# the walks rbh_test_trace has (its mode bits) over full boxes
-FULL_WALKS = {"four-wide": 0, "binary": 4, "four lanes": 16}
+# the walks rbh_test_trace has (its mode bits)
+WALKS = {"four-wide": 0, "binary": 4, "grid": 8, "four lanes": 16}
 
 
 @pytest.mark.parametrize("kind", ["nan", "infinity", "infinite-flat", "overflow"])
@@ -152,7 +152,7 @@ def test_vertices_that_are_not_finite(ctx, n, bad, kind):
             _upload(ctx, v, idx)
         b = _brute(v[:3 * n], idx[:n], rays, False)
         hit = b[:, 1].view(np.uint32) != 0xFFFFFFFF
-        for name, mode in FULL_WALKS.items():
+        for name, mode in WALKS.items():
             g = _trace_mode(ctx, rays, mode)
             assert np.array_equal(g[:, 1].view(np.uint32) != 0xFFFFFFFF, hit), name
             np.testing.assert_allclose(g[hit, 0], b[hit, 0], rtol=1e-5, atol=1e-5, err_msg=name)
