@@ -33,7 +33,8 @@ int rbh_test_oct(rbh_ctx ctx, const float* v, uint32_t* enc, float* dec, uint32_
  * global spill part of the traversal stack is exercised; bit 2: traverse the
  * binary tree instead of the four-wide one the renderer uses; bit 3: the
  * four-wide nodes with boxes on an 11-bit grid; bit 4: the four-wide walk with four
- * lanes per ray (its own 2-entry stack with bit 1). */
+ * lanes per ray, over either form of the nodes (its own 2-entry stack with
+ * bit 1). */
 int rbh_test_trace(rbh_ctx ctx, const float* rays, float* hits, uint32_t n, int mode);
 /* The built LBVH (replaces optixAccelBuild, rendering_interface.cpp:733-1064):
  * sorted 64-bit keys (Morton code << b | triangle, b the bits that hold n - 1,

@@ -89,8 +89,8 @@ __device__ __forceinline__ Bvh4HNode grid_node(const Bvh4Node& nd) {
         q.meta |= ((uint32_t)e & 0xFFu) << (8 * a);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            q.row[a][0][k] = grid_plane<false>(lo[k], o, e);
-            q.row[a][1][k] = grid_plane<true>(hi[k], o, e);
+            q.plane[k][a][0] = grid_plane<false>(lo[k], o, e);
+            q.plane[k][a][1] = grid_plane<true>(hi[k], o, e);
         }
     };
     axis(0, nd.lox, nd.hix);

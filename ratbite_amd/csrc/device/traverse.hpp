@@ -86,6 +86,11 @@ __device__ __forceinline__ bool tri_hit(const RayShear& s, V3 o, const TriRecord
 // resident per CU than a full 64-entry LDS stack would.
 constexpr int kMaxStack = 64;     // binary tree: depth <= 64
 constexpr int kMaxStack4 = 192;   // four-wide tree: at most 3 deferred children per level, <= 64 levels
+// Entries of the closest-hit walks with a distance (DistStack): six bytes each
+// in LDS, as many as leave room for seven waves per SIMD of the trace kernel,
+// which the registers allow. Every closest-hit walk keeps as many, so that
+// they drop the same entries.
+constexpr int kDistLds = 12;
 
 template <int LDS_DEPTH>
 struct TravStack {
@@ -237,7 +242,9 @@ __device__ __forceinline__ Hit traverse(const BvhNode* __restrict__ nodes, const
 struct TravRay {
     V3 o, d;
     float ix, iy, iz;
-    uint32_t ox, oy, oz;   // byte offset in a Bvh4Node of the row of near planes per axis
+    // per axis: byte offset in a Bvh4Node of the row of near planes; modulo 32
+    // the rotation that brings the near plane of a Bvh4HNode's pair down
+    uint32_t ox, oy, oz;
     RayShear sh;
     Hit h;
     int node;   // next node to visit (~i: the root is triangle i)
@@ -314,38 +321,78 @@ __device__ __forceinline__ void visit_node(const Bvh4Node* __restrict__ nodes, c
 // moved outwards by four units of its own size (2^-22), which covers them and
 // the rounding of the product's factor; the relative error of the sum is the
 // caller's margin.
+struct GridAxis {
+    float a, bn, bf;   // distance to near plane q: q a + bn, to far plane q: q a + bf
+};
+__device__ __forceinline__ GridAxis grid_axis(uint32_t meta, int sh, uint32_t corner, float o, float i) {
+    const float b = (__uint_as_float(corner) - o) * i;
+    return GridAxis{ldexpf(i, (int)(meta << (24 - sh)) >> 24), fmaf(fabsf(b), -2.3841858e-7f, b),
+                    fmaf(fabsf(b), 2.3841858e-7f, b)};
+}
+__device__ __forceinline__ float half_bits(uint32_t u) { return (float)__builtin_bit_cast(_Float16, (uint16_t)u); }
+// The pair of planes w of one slot and axis: near in tn, far in tf.
+__device__ __forceinline__ void grid_planes(const GridAxis& g, uint32_t w, uint32_t rotation, float& tn, float& tf) {
+    const uint32_t r = __builtin_rotateright32(w, rotation);
+    tn = fmaf(half_bits(r), g.a, g.bn);
+    tf = fmaf(half_bits(r >> 16), g.a, g.bf);
+}
+
 __device__ __forceinline__ void visit_node(const Bvh4HNode* __restrict__ nodes, const TravRay& r, Visit4& v) {
     const Bvh4HNode* __restrict__ nd = nodes + r.node;
     const uint4* q = reinterpret_cast<const uint4*>(nd);
-    const uint4 h = q[0], rx = q[1], ry = q[2], rz = q[3];
+    const uint4 h = q[0], p0 = q[1], p1 = q[2], p2 = q[3];
     v.first = (uint32_t)nd->child[0];
-    auto axis = [&](int sh, uint32_t ow, float o, float i, const uint4& w, float (&n)[4], float (&f)[4]) {
-        const float a = ldexpf(i, (int)(h.w << (24 - sh)) >> 24);
-        const float b = (__uint_as_float(ow) - o) * i;
-        const float bn = fmaf(fabsf(b), -2.3841858e-7f, b), bf = fmaf(fabsf(b), 2.3841858e-7f, b);
-        const bool neg = i < 0.0f;
-        const uint32_t n0 = neg ? w.z : w.x, n1 = neg ? w.w : w.y, f0 = neg ? w.x : w.z, f1 = neg ? w.y : w.w;
-        auto half = [](uint32_t u, int k) {
-            return (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> (16 * k)));
-        };
-        n[0] = fmaf(half(n0, 0), a, bn); n[1] = fmaf(half(n0, 1), a, bn);
-        n[2] = fmaf(half(n1, 0), a, bn); n[3] = fmaf(half(n1, 1), a, bn);
-        f[0] = fmaf(half(f0, 0), a, bf); f[1] = fmaf(half(f0, 1), a, bf);
-        f[2] = fmaf(half(f1, 0), a, bf); f[3] = fmaf(half(f1, 1), a, bf);
-    };
-    float nx[4], fx[4], ny[4], fy[4], nz[4], fz[4];
-    axis(0, h.x, r.o.x, r.ix, rx, nx, fx);
-    axis(8, h.y, r.o.y, r.iy, ry, ny, fy);
-    axis(16, h.z, r.o.z, r.iz, rz, nz, fz);
+    const uint32_t w[4][3] = {{p0.x, p0.y, p0.z}, {p0.w, p1.x, p1.y}, {p1.z, p1.w, p2.x}, {p2.y, p2.z, p2.w}};
+    const GridAxis x = grid_axis(h.w, 0, h.x, r.o.x, r.ix), y = grid_axis(h.w, 8, h.y, r.o.y, r.iy),
+                   z = grid_axis(h.w, 16, h.z, r.o.z, r.iz);
     v.tris = (h.w >> 24) & 15u;
     const uint32_t inner = h.w >> 28;
 #pragma unroll
     for (uint32_t k = 0; k < 4u; ++k) {
-        v.tn[k] = fmaxf(fmaxf(nx[k], ny[k]), nz[k]);
-        v.tf[k] = fminf(fminf(fx[k], fy[k]), fz[k]);
+        float nx, fx, ny, fy, nz, fz;
+        grid_planes(x, w[k][0], r.ox, nx, fx);
+        grid_planes(y, w[k][1], r.oy, ny, fy);
+        grid_planes(z, w[k][2], r.oz, nz, fz);
+        v.tn[k] = fmaxf(fmaxf(nx, ny), nz);
+        v.tf[k] = fminf(fminf(fx, fy), fz);
         v.order[k] = k < inner ? k : 4u;
     }
 }
+
+// The same for child k alone, by the same arithmetic: where the ray enters and
+// leaves its box (an empty slot has no meaningful distances), and the child's
+// reference.
+__device__ __forceinline__ int visit_child(const Bvh4Node* __restrict__ nodes, const TravRay& r, uint32_t k, float& tn,
+                                           float& tf) {
+    const Bvh4Node* __restrict__ nd = nodes + r.node;
+    const float* rows = reinterpret_cast<const float*>(nd) + k;
+    auto row = [&](uint32_t off) { return rows[off >> 2]; };
+    const float nx = row(r.ox), fx = row(r.ox ^ 16u), ny = row(r.oy), fy = row(r.oy ^ 16u), nz = row(r.oz), fz = row(r.oz ^ 16u);
+    tn = fmaxf(fmaxf((nx - r.o.x) * r.ix, (ny - r.o.y) * r.iy), (nz - r.o.z) * r.iz);
+    tf = fminf(fminf((fx - r.o.x) * r.ix, (fy - r.o.y) * r.iy), (fz - r.o.z) * r.iz);
+    return nd->child[k];
+}
+__device__ __forceinline__ int visit_child(const Bvh4HNode* __restrict__ nodes, const TravRay& r, uint32_t k, float& tn,
+                                           float& tf) {
+    const Bvh4HNode* __restrict__ nd = nodes + r.node;
+    const uint4 h = *reinterpret_cast<const uint4*>(nd);
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(nd->plane[k]);
+    float nx, fx, ny, fy, nz, fz;
+    grid_planes(grid_axis(h.w, 0, h.x, r.o.x, r.ix), w[0], r.ox, nx, fx);
+    grid_planes(grid_axis(h.w, 8, h.y, r.o.y, r.iy), w[1], r.oy, ny, fy);
+    grid_planes(grid_axis(h.w, 16, h.z, r.o.z, r.iz), w[2], r.oz, nz, fz);
+    tn = fmaxf(fmaxf(nx, ny), nz);
+    tf = fminf(fminf(fx, fy), fz);
+    return nd->child[k];
+}
+
+// The margins of a step: a box is met if it is entered before it is left and
+// before the hit so far, and visited if that hit, after the node's triangles,
+// still lies behind its entry.
+__device__ __forceinline__ bool box_met(float tn, float tf, float hit) {
+    return tn <= fminf(tf, hit * 1.00000024f) * 1.0000005f;
+}
+__device__ __forceinline__ float visit_limit(float hit) { return hit * 1.00000024f * 1.0000005f; }
 
 __device__ __forceinline__ uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
 __device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a < b ? b : a; }
@@ -384,13 +431,10 @@ __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const 
     visit_node(nodes, r, v);
     float tn[4];
     bool in[4];
-    {
-        const float best = r.h.t * 1.00000024f;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            tn[k] = fmaxf(v.tn[k], 0.0f);
-            in[k] = tn[k] <= fminf(v.tf[k], best) * 1.0000005f;
-        }
+    for (int k = 0; k < 4; ++k) {
+        tn[k] = fmaxf(v.tn[k], 0.0f);
+        in[k] = box_met(tn[k], v.tf[k], r.h.t);
     }
     // Triangle children first (a hit shortens the ray for the boxes), in
     // slot order. One loop over each lane's own triangle slots: a wave runs
@@ -420,7 +464,7 @@ __device__ __forceinline__ bool trav_step(const NODE* __restrict__ nodes, const 
     // inner children in the two low bits: their indices are consecutive, and
     // children within 4 ulp of each other go in slot order. Culled and empty
     // slots sort last as ~0.
-    const float limit = r.h.t * 1.00000024f * 1.0000005f;
+    const float limit = visit_limit(r.h.t);
     uint32_t key[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)

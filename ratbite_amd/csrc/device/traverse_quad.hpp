@@ -6,9 +6,11 @@
 // waves per SIMD. (With the chip full it is slower: the same boxes cost four
 // times the lanes and the ordering work is repeated by every lane.)
 //
-// The walk is the per-lane one exactly: children in the same order, triangle
-// tests folded in slot order with the same comparisons, so closest hits are
-// the same bits whichever form ran, ties included.
+// The walk is trav_step's: the same node form, the same arithmetic per box and
+// margins, triangle tests folded in slot order with the same comparisons,
+// children visited in the same order and deferred ones dropped by the same
+// distances. So hits are the same bits whichever form ran over the same nodes,
+// ties included.
 #pragma once
 #include "traverse.hpp"
 
@@ -16,7 +18,7 @@ namespace rbh {
 namespace dev {
 
 constexpr int kQuadRays = 16;      // rays of a wave
-constexpr int kQuadStackLds = 64;  // stack entries per ray in LDS (4 KB per wave); deeper ones spill
+constexpr int kQuadStackLds = 64;  // stack entries per ray in LDS (8 KB per wave); deeper ones spill
 
 // The value of lane J of the quad / of the quad's lane xor X, on all four lanes.
 template <int J>
@@ -31,10 +33,29 @@ __device__ __forceinline__ uint32_t quad_xor(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
 }
 
-// Row r (lo x, hi x, lo y, hi y, lo z, hi z, child) of child j of a node.
-__device__ __forceinline__ float node_row(const Bvh4Node* __restrict__ n, int r, uint32_t j) {
-    return reinterpret_cast<const float*>(n)[4 * r + (int)j];
-}
+// The stack of a ray's quad: LDS_DEPTH entries in LDS with the key they were
+// deferred under, read together, and deeper ones in the spill column. Entries
+// from DIST_DEPTH on are visited whatever their distance, as DistStack's are.
+template <int LDS_DEPTH, int DIST_DEPTH>
+struct QuadStack {
+    uint2* __restrict__ lds;
+    int stride;
+    int* __restrict__ spill;
+    uint32_t spillStride;
+    __device__ __forceinline__ void put(int sp, int v, uint32_t key) const {
+        if (sp < LDS_DEPTH) lds[sp * stride] = make_uint2((uint32_t)v, key);
+        else spill[(size_t)(sp - LDS_DEPTH) * spillStride] = v;
+    }
+    // Entry sp; beyond: it starts after distance `limit` (its distance cut to
+    // the 16 bits that DistStack keeps).
+    __device__ __forceinline__ int get(int sp, float limit, bool& beyond) const {
+        beyond = false;
+        if (sp >= LDS_DEPTH) return spill[(size_t)(sp - LDS_DEPTH) * spillStride];
+        const uint2 e = lds[sp * stride];
+        beyond = sp < DIST_DEPTH && __uint_as_float(e.y & 0xFFFF0000u) > limit;
+        return (int)e.x;
+    }
+};
 
 // One fold step of the closest hit: lane K's candidate against the ray's
 // distance so far, as tri_hit compares it.
@@ -52,42 +73,32 @@ __device__ __forceinline__ void quad_fold(bool cand, float T, float det, float t
 // The closest hit below tmax or, with ANY, whether there is one (leaf other
 // than ~0). All four lanes of a quad pass the same ray and receive the same
 // hit; quads of a wave may be inactive as a whole.
-template <bool ANY, int LDS_DEPTH>
-__device__ __forceinline__ Hit traverse4_quad(const Bvh4Node* __restrict__ nodes, const TriRecord* __restrict__ tris,
-                                              uint32_t nnodes, V3 o, V3 d, float tmax,
-                                              const TravStack<LDS_DEPTH>& stack) {
+template <bool ANY, typename STACK, typename NODE>
+__device__ __forceinline__ Hit traverse4_quad(const NODE* __restrict__ nodes, const TriRecord* __restrict__ tris,
+                                              uint32_t nnodes, V3 o, V3 d, float tmax, const STACK& stack) {
     const uint32_t j = (uint32_t)__lane_id() & 3u;
-    Hit h;
-    h.t = tmax;
-    h.leaf = 0xFFFFFFFFu;
-    h.b1 = h.b2 = 0.0f;
-    const RayShear sh = make_shear(d);
+    TravRay r;
+    trav_init(r, o, d, tmax, nnodes);
+    Hit& h = r.h;
     if (nnodes == 0u) {
         // a single-triangle scene
         float t, b1, b2;
-        if (tri_hit(sh, o, tris[0], tmax, t, b1, b2)) h = Hit{t, b1, b2, 0u};
+        if (tri_hit(r.sh, o, tris[0], tmax, t, b1, b2)) h = Hit{t, b1, b2, 0u};
         return h;
     }
-    const float ix = 1.0f / d.x, iy = 1.0f / d.y, iz = 1.0f / d.z;
     // this lane's last accepted triangle; owner: the quad lane holding the closest hit (4: none)
     float mb1 = 0.0f, mb2 = 0.0f;
     uint32_t mleaf = 0u, owner = 4u;
-    int node = 0, sp = 0;
     while (true) {
-        const Bvh4Node* __restrict__ n = nodes + node;
-        const float lx = node_row(n, 0, j), hx = node_row(n, 1, j), ly = node_row(n, 2, j), hy = node_row(n, 3, j),
-                    lz = node_row(n, 4, j), hz = node_row(n, 5, j);
-        const int ch = (int)__float_as_uint(node_row(n, 6, j));
-        const float best = h.t * 1.00000024f;
-        const float x0 = (lx - o.x) * ix, x1 = (hx - o.x) * ix;
-        const float y0 = (ly - o.y) * iy, y1 = (hy - o.y) * iy;
-        const float z0 = (lz - o.z) * iz, z1 = (hz - o.z) * iz;
-        const float tnear = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
-        const float tfar = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), best));
-        const bool in = ch != kBvh4Empty && tnear <= tfar * 1.00000024f;
+        float tn, tf;
+        const int ch = visit_child(nodes, r, j, tn, tf);
+        tn = fmaxf(tn, 0.0f);
+        const bool in = ch != kBvh4Empty && box_met(tn, tf, h.t);
         bool cand = false;
         float T = 0.0f, det = 0.0f, t = 0.0f, b1 = 0.0f, b2 = 0.0f;
-        if (in && ch < 0) cand = tri_candidate(sh, o, tris[~ch], h.t, T, det, t, b1, b2);
+        // (closest hit: the distance is compared in the fold alone, as an accepted
+        // hit may lie a rounding behind the one before it)
+        if (in && ch < 0) cand = tri_candidate(r.sh, o, tris[~ch], ANY ? h.t : INFINITY, T, det, t, b1, b2);
         if (__ballot(cand) != 0ull) {
             if (ANY) {
                 const uint32_t c = cand ? 1u : 0u;
@@ -112,25 +123,28 @@ __device__ __forceinline__ Hit traverse4_quad(const Bvh4Node* __restrict__ nodes
             }
         }
         // surviving inner children nearest first, ordered by the keys of the per-lane walk
-        const float limit = h.t * 1.00000024f * 1.00000024f;
-        const uint32_t key = (in && ch >= 0 && tnear <= limit) ? ((__float_as_uint(tnear) & 0x7FFFFFFCu) | j) : ~0u;
+        const float limit = visit_limit(h.t);
+        const uint32_t key = (in && ch >= 0 && (ANY || tn <= limit)) ? ((__float_as_uint(tn) & 0x7FFFFFFCu) | j) : ~0u;
         const uint32_t k1 = quad_xor<1>(key), k2 = quad_xor<2>(key), k3 = quad_xor<3>(key);
         const uint32_t rank = (k1 < key ? 1u : 0u) + (k2 < key ? 1u : 0u) + (k3 < key ? 1u : 0u);
         const uint32_t cnt = (key != ~0u ? 1u : 0u) + (k1 != ~0u ? 1u : 0u) + (k2 != ~0u ? 1u : 0u) + (k3 != ~0u ? 1u : 0u);
         if (cnt != 0u) {
             // the nearest next, the others farthest first on the stack
-            if (key != ~0u && rank != 0u) stack.put(sp + (int)(cnt - 1u - rank), ch);
+            if (key != ~0u && rank != 0u) stack.put(r.sp + (int)(cnt - 1u - rank), ch, key);
             uint32_t next = key != ~0u && rank == 0u ? (uint32_t)ch : 0u;
             next |= quad_xor<1>(next);
             next |= quad_xor<2>(next);
-            node = (int)next;
-            sp += (int)cnt - 1;
+            r.node = (int)next;
+            r.sp += (int)cnt - 1;
             continue;
         }
-        if (sp == 0) break;
-        --sp;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // the entry may be another lane's
-        node = stack.get(sp);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // the entries may be another lane's
+        bool beyond = true;
+        while (beyond && r.sp > 0) {
+            r.node = stack.get(--r.sp, limit, beyond);
+            if (ANY) beyond = false;
+        }
+        if (beyond) break;
     }
     if (!ANY && owner != 4u) {
         const int src = (__lane_id() & ~3) | (int)owner;

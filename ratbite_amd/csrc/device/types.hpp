@@ -55,7 +55,7 @@ constexpr uint32_t kMaxNodes4 = 1u << 25;
 struct alignas(128) Bvh4HNode {
     float o[3];
     uint32_t meta;           // e per axis as signed bytes (x lowest), bits 24-27 slots with a triangle, 28-30 number of inner children
-    uint16_t row[3][2][4];   // per axis: the lower planes of the four slots, the upper ones (half floats; empty slot: +inf, -inf)
+    uint16_t plane[4][3][2]; // per slot and axis: the lower and the upper plane (half floats; empty slot: +inf, -inf)
     int32_t child[4];        // as in Bvh4Node
     int32_t pad[12];
 };

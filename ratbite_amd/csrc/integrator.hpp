@@ -117,6 +117,7 @@ struct Frame1 {
     uint32_t bounce;
     uint32_t camOrigin0;          // no scene of the pass uses depth of field: camera rays start at 0
     uint32_t sortHits;            // LaunchShape::sortHits
+    uint32_t gridNodes;           // the pass's walks read the nodes on an 11-bit grid
     uint32_t tail;                // queues of at most so many paths are run to their end by k_paths (0: none)
     // state
     PathBuffers p;

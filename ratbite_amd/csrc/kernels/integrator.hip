@@ -37,11 +37,8 @@ using namespace wf;
 
 namespace {
 
-// Traversal stack entries kept in LDS per lane: of the any-hit walk, and of
-// the closest-hit walk with their distances (6 bytes each), as many as leave
-// room for the seven waves per SIMD that the registers allow
+// Traversal stack entries of the any-hit walk kept in LDS per lane
 constexpr int kStackLds = 16;
-constexpr int kDistLds = 12;
 
 __device__ __forceinline__ uint32_t wave_push(uint32_t* __restrict__ counter, bool pred) {
     // one atomic per wave: ballot, leader adds the popcount, lanes take
@@ -477,9 +474,9 @@ __global__ __launch_bounds__(kShadeBlock, WAVES) void k_shade(Frame1 f, uint32_t
 // each of them (about 200 us however few the paths); here a wave only waits
 // for its own 16 paths, and their walks take one box and one triangle per
 // lane (traverse_quad.hpp). The four lanes shade their path redundantly, with
-// the same values, and only the first one counts. State and per-path bodies
-// are those of the separate kernels, so a path's values do not depend on
-// which form ran it. Bound by the latency of a path's chain of bounces: one
+// the same values, and only the first one counts. State, per-path bodies, node
+// form and walk are those of the separate kernels, so a path's values do not
+// depend on which form ran it. Bound by the latency of a path's chain of bounces: one
 // sample of a 64x64 Cornell box at depth 8 takes 0.42 ms against 1.27 ms in
 // the separate kernels (0.68 ms with one lane per path), 640x360 over 1M
 // triangles with a refit 3.9 against 5.3 ms. bounce: the bounce the queue
@@ -498,9 +495,9 @@ constexpr int kTailWaves = 3;
 constexpr uint32_t kFewPaths = 32768u;
 template <bool BATCH, int WAVES>
 __global__ __launch_bounds__(kPathBlock, WAVES) void k_paths(Frame1 f, uint32_t bounce, uint32_t depthMax) {
-    __shared__ int stack[kQuadStackLds * kQuadRays];
+    __shared__ uint2 stack[kQuadStackLds * kQuadRays];
     const uint32_t t = (blockIdx.x * kPathBlock + threadIdx.x) >> 2;
-    const TravStack<kQuadStackLds> st{stack + (threadIdx.x >> 2), kQuadRays, f.spill + t, f.spillStride};
+    const QuadStack<kQuadStackLds, kDistLds> st{stack + (threadIdx.x >> 2), kQuadRays, f.spill + t, f.spillStride};
     const uint32_t qsel = bounce & 1u;
     const uint32_t count = f.counters[qsel ? CNT_QUEUE1 : CNT_QUEUE0];
     if (count > f.tail) return;   // long enough for the separate kernels
@@ -516,7 +513,8 @@ __global__ __launch_bounds__(kPathBlock, WAVES) void k_paths(Frame1 f, uint32_t 
             float ts = 3.402823466e+38f;
             uint32_t shape = 0xFFFFFFFFu;
             if (S.nshapes) shape_closest(S.shapes, S.nshapes, o, d, ts, ts, shape);
-            Hit h = traverse4_quad<false>(S.nodes4, S.tris, S.nnodes4, o, d, ts, st);
+            Hit h = f.gridNodes ? traverse4_quad<false>(S.nodes4h, S.tris, S.nnodes4, o, d, ts, st)
+                                 : traverse4_quad<false>(S.nodes4, S.tris, S.nnodes4, o, d, ts, st);
             if (h.leaf == 0xFFFFFFFFu && shape != 0xFFFFFFFFu) h = Hit{ts, 0.0f, 0.0f, shape};
             ++nclosest;
             alive = false;
@@ -534,9 +532,11 @@ __global__ __launch_bounds__(kPathBlock, WAVES) void k_paths(Frame1 f, uint32_t 
             if (shadow) {
                 const float4 so = f.p.sro[pid], sd = f.p.srd[pid];
                 const V3 so3{so.x, so.y, so.z}, sd3{sd.x, sd.y, sd.z};
-                if (!(S.nshapes && shape_any(S.shapes, S.nshapes, so3, sd3, so.w)) &&
-                    traverse4_quad<true>(S.nodes4, S.tris, S.nnodes4, so3, sd3, so.w, st).leaf == 0xFFFFFFFFu)
-                    add_nee(f, pid);
+                if (!(S.nshapes && shape_any(S.shapes, S.nshapes, so3, sd3, so.w))) {
+                    const Hit q = f.gridNodes ? traverse4_quad<true>(S.nodes4h, S.tris, S.nnodes4, so3, sd3, so.w, st)
+                                              : traverse4_quad<true>(S.nodes4, S.tris, S.nnodes4, so3, sd3, so.w, st);
+                    if (q.leaf == 0xFFFFFFFFu) add_nee(f, pid);
+                }
                 ++nshadow;
             }
         }
@@ -605,11 +605,15 @@ static void launch_trace_q(rbh_ctx c, const Frame1& f, uint32_t qsel, const Laun
 }
 
 // The work-fetch variants read the nodes with full boxes, which are indexed
-// up to 4 GiB; larger trees run the nodes on the grid.
+// up to 4 GiB; larger trees run the nodes on the grid. All kernels of a pass
+// read the same form.
+static bool work_fetch(const LaunchShape& ls) { return ls.traceFetch && !ls.quantOnly; }
+static bool grid_nodes(const LaunchShape& ls) { return ls.quantOnly || (ls.quantNodes && !ls.traceFetch); }
+
 template <bool BATCH>
 static void launch_trace(rbh_ctx c, const Frame1& f, uint32_t qsel, const LaunchShape& ls) {
-    if (ls.traceFetch && !ls.quantOnly) launch_trace_q<BATCH, true, false>(c, f, qsel, ls);
-    else if (ls.quantNodes || ls.quantOnly) launch_trace_q<BATCH, false, true>(c, f, qsel, ls);
+    if (work_fetch(ls)) launch_trace_q<BATCH, true, false>(c, f, qsel, ls);
+    else if (grid_nodes(ls)) launch_trace_q<BATCH, false, true>(c, f, qsel, ls);
     else launch_trace_q<BATCH, false, false>(c, f, qsel, ls);
 }
 
@@ -623,8 +627,8 @@ static void launch_shadow_q(rbh_ctx c, const Frame1& f, const LaunchShape& ls) {
 
 template <bool BATCH>
 static void launch_shadow(rbh_ctx c, const Frame1& f, const LaunchShape& ls) {
-    if (ls.traceFetch && !ls.quantOnly) launch_shadow_q<BATCH, true, false>(c, f, ls);
-    else if (ls.quantNodes || ls.quantOnly) launch_shadow_q<BATCH, false, true>(c, f, ls);
+    if (work_fetch(ls)) launch_shadow_q<BATCH, true, false>(c, f, ls);
+    else if (grid_nodes(ls)) launch_shadow_q<BATCH, false, true>(c, f, ls);
     else launch_shadow_q<BATCH, false, false>(c, f, ls);
 }
 
@@ -650,6 +654,7 @@ static hipError_t launch_pass_t(rbh_ctx c, Frame1 f, uint32_t depthMax, const La
     } while (0)
     f.bounce = 0;
     f.sortHits = ls.sortHits ? 1u : 0u;
+    f.gridNodes = grid_nodes(ls) ? 1u : 0u;
     uint32_t* const counters = f.counters;
     const uint32_t ncount = (depthMax + 1u) * CNT_COUNT;
     hipLaunchKernelGGL(k_pass_start, dim3((ncount + 255u) / 256u), dim3(256), 0, c->stream, f, ncount);
@@ -661,16 +666,17 @@ static hipError_t launch_pass_t(rbh_ctx c, Frame1 f, uint32_t depthMax, const La
     const dim3 pathGrid(std::min<uint32_t>((std::min(std::max(f.tail, 1u), f.NP) + kQuadRays - 1) / kQuadRays,
                                            (uint32_t)ls.traceGrid * kTraceBlock / kQuadRays));
     const bool allPaths = f.NP <= f.tail;
-    if (allPaths && f.NP <= kFewPaths)
-        hipLaunchKernelGGL((k_paths<BATCH, 2>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
-    else if (allPaths)
-        hipLaunchKernelGGL((k_paths<BATCH, kTailWaves>), pathGrid, dim3(kPathBlock), 0, c->stream, f, 0u, depthMax);
+    const auto paths = [&](uint32_t b) {
+        const bool few = b == 0u && f.NP <= kFewPaths;
+        auto k = few ? k_paths<BATCH, 2> : k_paths<BATCH, kTailWaves>;
+        hipLaunchKernelGGL(k, pathGrid, dim3(kPathBlock), 0, c->stream, f, b, depthMax);
+    };
+    if (allPaths) paths(0u);
     for (uint32_t b = 0; b < depthMax && !allPaths; ++b) {
         const uint32_t qsel = b & 1u;
         f.bounce = b;
         f.counters = counters + b * CNT_COUNT;
-        if (f.tail && b > 0)
-            hipLaunchKernelGGL((k_paths<BATCH, kTailWaves>), pathGrid, dim3(kPathBlock), 0, c->stream, f, b, depthMax);
+        if (f.tail && b > 0) paths(b);
         RBH_TIMED(KernelTimer::TRACE, launch_trace<BATCH>(c, f, qsel, ls));
         RBH_TIMED(KernelTimer::SHADE,
                   hipLaunchKernelGGL(k_miss<BATCH>, dim3(ls.shadeGrid), dim3(256), 0, c->stream, f));

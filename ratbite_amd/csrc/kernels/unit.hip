@@ -87,9 +87,20 @@ __global__ __launch_bounds__(128) void k_trace_test(const BvhNode* nodes, const 
     const TravStack<LDS_DEPTH> st{stack + threadIdx.x, 128, spill + i, spillStride};
     const float* r = rays + 8 * (size_t)i;
     const V3 ro{r[0], r[1], r[2]}, rd{r[4], r[5], r[6]};
-    const Hit h = tree == 1 ? traverse<ANY>(nodes, tris, nnodes, ro, rd, r[7], st)
-                : tree == 2 ? traverse4<ANY>(nodes4h, tris, nnodes4, ro, rd, r[7], st)
-                            : traverse4<ANY>(nodes4, tris, nnodes4, ro, rd, r[7], st);
+    Hit h;
+    if (tree == 1) {
+        h = traverse<ANY>(nodes, tris, nnodes, ro, rd, r[7], st);
+    } else {
+        // the renderer's stacks: with distances in the closest-hit walks
+        constexpr int D = LDS_DEPTH < kDistLds ? LDS_DEPTH : kDistLds;
+        __shared__ uint16_t dist[ANY ? 1 : D * 128];
+        const auto walk = [&](const auto& stack4) {
+            return tree == 2 ? traverse4<ANY>(nodes4h, tris, nnodes4, ro, rd, r[7], stack4)
+                             : traverse4<ANY>(nodes4, tris, nnodes4, ro, rd, r[7], stack4);
+        };
+        if constexpr (ANY) h = walk(st);
+        else h = walk(DistStack<D>{stack + threadIdx.x, dist + threadIdx.x, 128, spill + i, spillStride});
+    }
     float* o = hits + 4 * (size_t)i;
     o[0] = h.leaf == 0xFFFFFFFFu ? -1.0f : h.t;
     o[1] = __uint_as_float(h.leaf == 0xFFFFFFFFu ? 0xFFFFFFFFu : tris[h.leaf].prim);
@@ -98,14 +109,15 @@ __global__ __launch_bounds__(128) void k_trace_test(const BvhNode* nodes, const 
 }
 
 // the four-lanes-per-ray walk, 32 rays per block
-template <bool ANY, int LDS_DEPTH>
-__global__ __launch_bounds__(128) void k_trace_quad_test(const Bvh4Node* nodes4, const TriRecord* tris, uint32_t nn4,
+template <bool ANY, int LDS_DEPTH, typename NODE>
+__global__ __launch_bounds__(128) void k_trace_quad_test(const NODE* nodes4, const TriRecord* tris, uint32_t nn4,
                                                          const float* rays, float* hits, uint32_t n, int* spill,
                                                          uint32_t spillStride) {
-    __shared__ int stack[LDS_DEPTH * 32];
+    constexpr int D = LDS_DEPTH < kDistLds ? LDS_DEPTH : kDistLds;
+    __shared__ uint2 stack[LDS_DEPTH * 32];
     const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 2;
     if (i >= n) return;
-    const TravStack<LDS_DEPTH> st{stack + (threadIdx.x >> 2), 32, spill + i, spillStride};
+    const QuadStack<LDS_DEPTH, D> st{stack + (threadIdx.x >> 2), 32, spill + i, spillStride};
     const float* r = rays + 8 * (size_t)i;
     const Hit h = traverse4_quad<ANY>(nodes4, tris, nn4, V3{r[0], r[1], r[2]}, V3{r[4], r[5], r[6]}, r[7], st);
     if (threadIdx.x & 3u) return;
@@ -319,9 +331,14 @@ int rbh_test_trace(rbh_ctx c, const float* rays, float* hits, uint32_t n, int mo
         const uint32_t cols = gq.x * 32u;
         int* sq = (int*)s.out((size_t)cols * kMaxStack4 * 4);
         STAGE_CHECK(sq);
-        auto k = any ? (tiny ? k_trace_quad_test<true, 2> : k_trace_quad_test<true, kQuadStackLds>)
-                     : (tiny ? k_trace_quad_test<false, 2> : k_trace_quad_test<false, kQuadStackLds>);
-        hipLaunchKernelGGL(k, gq, dim3(128), 0, 0, nodes4, tris, nn4, (const float*)dr, (float*)dh, n, sq, cols);
+        const auto launch = [&](const auto* nodes) {
+            using N = std::remove_cv_t<std::remove_pointer_t<decltype(nodes)>>;
+            auto k = any ? (tiny ? k_trace_quad_test<true, 2, N> : k_trace_quad_test<true, kQuadStackLds, N>)
+                         : (tiny ? k_trace_quad_test<false, 2, N> : k_trace_quad_test<false, kQuadStackLds, N>);
+            hipLaunchKernelGGL(k, gq, dim3(128), 0, 0, nodes, tris, nn4, (const float*)dr, (float*)dh, n, sq, cols);
+        };
+        if (mode & 8) launch(nodes4h);
+        else launch(nodes4);
         FINISH(hits, dh, (size_t)n * 16);
         return RBH_OK;
     }

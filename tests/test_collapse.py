@@ -16,7 +16,7 @@ import host_wavefront as H  # noqa: E402
 
 EMPTY = -2 ** 31
 NODE4_DTYPE = np.dtype([(k, "f4", 4) for k in ("lox", "hix", "loy", "hiy", "loz", "hiz")] + [("child", "i4", 4), ("pad", "i4", 4)])
-NODE4H_DTYPE = np.dtype([("o", "f4", 3), ("meta", "u4"), ("row", "f2", (3, 2, 4)), ("child", "i4", 4), ("pad", "i4", 12)])
+NODE4H_DTYPE = np.dtype([("o", "f4", 3), ("meta", "u4"), ("plane", "f2", (4, 3, 2)), ("child", "i4", 4), ("pad", "i4", 12)])
 
 
 @pytest.fixture(scope="module")
@@ -117,8 +117,8 @@ def test_grid_boxes_hold_the_full_ones(lib, kind):
             e = ((n4h["meta"] >> np.uint32(8 * a)) & np.uint32(0xFF)).astype(np.int8).astype(np.float64)
             with np.errstate(invalid="ignore"):
                 plane = n4h["o"][:, a, None, None].astype(np.float64) + \
-                    n4h["row"][:, a].astype(np.float64) * np.exp2(e)[:, None, None]
-            below, above = plane[:, 0][full], plane[:, 1][full]
+                    n4h["plane"][:, :, a].astype(np.float64) * np.exp2(e)[:, None, None]
+            below, above = plane[..., 0][full], plane[..., 1][full]
             l, h = n4[lo][full].astype(np.float64), n4[hi][full].astype(np.float64)
             none = np.isnan(l)
             assert np.array_equal(none, np.isnan(h))
