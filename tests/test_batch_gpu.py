@@ -124,6 +124,17 @@ def test_autotune_keeps_results(ctx):
     r.set_tuning()
 
 
+def test_set_tuning_without_arguments_is_the_librarys_own():
+    import ratbite_amd
+    with ratbite_amd.Context(0) as c:
+        r = Renderer(scenes.cornell(width=8, height=8, spp=1), ctx=c)
+        own = r.tuning()
+        r.set_tuning(trace_blocks=64)
+        assert r.tuning() == dict(own, traceBlocksPerCU=64)
+        r.set_tuning()
+        assert r.tuning() == own
+
+
 def test_material_sorted_shading_keeps_results(ctx):
     # conductor hits queued from the end of the hit queue: the same sums for
     # plain, guided (the network's mixtures are indexed by queue position)
