@@ -154,7 +154,7 @@ typedef struct rbh_stats {
     double shadeMs;               /* time in shading kernels */
     double cdfMs;                 /* time of the last env-map CDF build kernel */
     double bvhMs;                 /* time of the last LBVH build */
-    uint32_t traceLaunches;       /* closest-hit kernel launches of the last render */
+    uint32_t traceLaunches;       /* bounces of the last render's passes (their closest-hit launches where no queue was short) */
     uint32_t bvhDepth;            /* max depth of the LBVH */
     double guideMs;               /* time in guiding inference kernels */
     uint64_t nonFiniteSamples;    /* samples whose radiance was not finite (added as black; the reference would
@@ -354,11 +354,13 @@ typedef struct rbh_tuning {
     int32_t quantNodes;           /* 1: the wave-synchronous trace/shadow kernels read the four-wide nodes with child boxes on an 11-bit grid (the default) */
     int32_t sortHits;             /* 1: material-sorted shading (hits queued by shading class: plain, transmissive and sheen
                                      ComplexSurface, PureConductor, PureDielectric, shape light) */
-    double samplesPerSecond;      /* measured by rbh_autotune */
+    double samplesPerSecond;      /* measured by rbh_autotune, every bounce in the per-bounce kernels */
 } rbh_tuning;
 /* Times trialSpp-sample renders of lp over a grid of slot budgets and grid
  * sizes, keeps the fastest on the context and returns it. Overwrites the
- * accumulation buffer. */
+ * accumulation buffer. The trials run the per-bounce kernels only, whose
+ * launch shapes these are (other renders run queues of at most 65536 paths in
+ * one kernel that has none of these settings but the nodes' form). */
 int rbh_autotune(rbh_ctx ctx, const rbh_launch_params* lp, uint32_t trialSpp, rbh_tuning* best);
 int rbh_set_tuning(rbh_ctx ctx, const rbh_tuning* t);
 /* The launch shape the context renders with (samplesPerSecond 0). */

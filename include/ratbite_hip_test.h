@@ -36,6 +36,11 @@ int rbh_test_oct(rbh_ctx ctx, const float* v, uint32_t* enc, float* dec, uint32_
  * lanes per ray, over either form of the nodes (its own 2-entry stack with
  * bit 1). */
 int rbh_test_trace(rbh_ctx ctx, const float* rays, float* hits, uint32_t n, int mode);
+/* Which bounces of the last pass ran in the per-bounce kernels (no reference
+ * counterpart): queued[b] = paths whose closest hit they queued at bounce b as
+ * hit or miss; 0 where the kernel for short queues ran. bounces <= 1024, and
+ * at most the last render's maxPathDepth hold values of that render. */
+int rbh_test_queued(rbh_ctx ctx, uint32_t* queued, uint32_t bounces);
 /* The built LBVH (replaces optixAccelBuild, rendering_interface.cpp:733-1064):
  * sorted 64-bit keys (Morton code << b | triangle, b the bits that hold n - 1,
  * the Morton code min(21, (64 - b) / 3) bits per axis), n entries; 64-byte nodes

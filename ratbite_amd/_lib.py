@@ -244,6 +244,7 @@ register({
     "rbh_test_lbvh_read": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, ctypes.POINTER(c_uint32)]),
     "rbh_test_radix_sort": (c_int, [c_void_p, c_void_p, c_void_p, c_uint32, c_int, c_int, c_void_p, c_void_p]),
     "rbh_test_select_positive": (c_int, [c_void_p, c_void_p, c_uint32, c_void_p, ctypes.POINTER(c_uint32)]),
+    "rbh_test_queued": (c_int, [c_void_p, c_void_p, c_uint32]),
     "rbh_test_trace": (c_int, [c_void_p, c_void_p, c_void_p, c_uint32, c_int]),
     "rbh_test_light_pdf": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32]),
     "rbh_test_light_sample": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32]),

@@ -155,6 +155,8 @@ struct RenderState {
     int traceWaves = 7;          // trace/shadow register budget (1, 7, 8 waves per SIMD)
     int quantNodes = 1;          // traverse the four-wide nodes with boxes on an 11-bit grid
     int sortHits = 1;            // shade conductor hits as their own run of the hit queue
+    bool tail = true;            // short queues run to their end in one kernel (off while the shapes of the others are timed)
+    const uint32_t* counters = nullptr;   // of the last pass, in paths
     DevBuf sceneTable;           // batched passes: SceneView per scene and pass
     bool useGraph = false;       // replay each pass's launch sequence as a captured HIP graph
     hipGraphExec_t graphExec = nullptr;

@@ -106,6 +106,7 @@ struct LaunchShape {
     int quantNodes;          // wave-synchronous trace/shadow kernels read the nodes on an 11-bit grid
     bool quantOnly;          // a tree of the pass is too large for the nodes with full boxes
     int sortHits;            // queue the hits by shading class (material-sorted shading)
+    bool tail;               // short queues run to their end in one kernel
 };
 
 struct Frame1 {

@@ -660,8 +660,9 @@ static hipError_t launch_pass_t(rbh_ctx c, Frame1 f, uint32_t depthMax, const La
     hipLaunchKernelGGL(k_pass_start, dim3((ncount + 255u) / 256u), dim3(256), 0, c->stream, f, ncount);
     // k_paths: launched before each later bounce of an unguided pass, it leaves
     // at once unless the queue has become short; a pass short from the start
-    // is that one launch. Per-kernel timing keeps the kernels apart.
-    f.tail = f.guided || kt ? 0u : kTailPaths;
+    // is that one launch. Per-kernel timing keeps the kernels apart, and so
+    // does the tuning of their shapes.
+    f.tail = f.guided || kt || !ls.tail ? 0u : kTailPaths;
     // (no more lanes than the trace grid's spill columns)
     const dim3 pathGrid(std::min<uint32_t>((std::min(std::max(f.tail, 1u), f.NP) + kQuadRays - 1) / kQuadRays,
                                            (uint32_t)ls.traceGrid * kTraceBlock / kQuadRays));

@@ -20,6 +20,7 @@
 #include "../device/qrng.hpp"
 #include "../device/traverse.hpp"
 #include "../device/traverse_quad.hpp"
+#include "../integrator.hpp"
 #include "radix.hpp"
 
 namespace rbh {
@@ -306,6 +307,19 @@ int rbh_test_oct(rbh_ctx c, const float* v, uint32_t* enc, float* dec, uint32_t 
     hipLaunchKernelGGL(k_oct, grid(n, 256), dim3(256), 0, 0, (const float*)dv, (uint32_t*)de, (float*)dd, n);
     FINISH(enc, de, (size_t)n * 4);
     RBH_HIP(c, hipMemcpy(dec, dd, (size_t)n * 12, hipMemcpyDeviceToHost));
+    return RBH_OK;
+}
+
+int rbh_test_queued(rbh_ctx c, uint32_t* queued, uint32_t bounces) {
+    if (!c || !queued || bounces > kMaxDepth) return RBH_ERR_INVALID;
+    if (!c->rs.counters) return fail(c, RBH_ERR_STATE, "nothing rendered");
+    std::vector<uint32_t> cnt((size_t)bounces * CNT_COUNT);
+    RBH_HIP(c, hipStreamSynchronize(c->stream));
+    RBH_HIP(c, hipMemcpy(cnt.data(), c->rs.counters, cnt.size() * 4, hipMemcpyDeviceToHost));
+    for (uint32_t b = 0; b < bounces; ++b) {
+        queued[b] = cnt[b * CNT_COUNT + CNT_MISS];
+        for (uint32_t k = 0; k < kShadeClasses; ++k) queued[b] += cnt[b * CNT_COUNT + hit_counter(k)];
+    }
     return RBH_OK;
 }
 

@@ -499,11 +499,13 @@ int prepare_pass_state(rbh_ctx c, size_t NP, Frame1& f, LaunchShape& ls) {
     uint32_t* counters = nullptr;
     unsigned long long* stats = nullptr;
     const size_t bytes = layout_paths(nullptr, NP, &pb, &counters, &stats);
+    rs.counters = nullptr;
     RBH_ALLOC(c, rs.paths, bytes);
     layout_paths(rs.paths.as<char>(), NP, &pb, &counters, &stats);
     f.p = pb;
     f.counters = counters;
     f.stats = stats;
+    rs.counters = counters;
     const int cus = cu_count(c->device);
     // persistent grids, never more lanes than the pass has path slots
     ls.traceGrid = (int)std::max<size_t>(1, std::min<size_t>((size_t)cus * rs.traceBlocksPerCU, (NP + kTraceBlock - 1) / kTraceBlock));
@@ -514,6 +516,7 @@ int prepare_pass_state(rbh_ctx c, size_t NP, Frame1& f, LaunchShape& ls) {
     ls.quantNodes = rs.quantNodes;
     ls.quantOnly = false;
     ls.sortHits = rs.sortHits;
+    ls.tail = rs.tail;
     const size_t lanes = (size_t)ls.traceGrid * kTraceBlock;
     RBH_ALLOC(c, rs.spill, trace_spill_words(lanes) * sizeof(int));
     f.spill = rs.spill.as<int>();
@@ -842,6 +845,13 @@ int rbh_autotune(rbh_ctx c, const rbh_launch_params* lp, uint32_t trialSpp, rbh_
     (void)freeB;
     const int keepF = rs.traceFetch, keepW = rs.shadeWaves, keepTW = rs.traceWaves, keepQ = rs.quantNodes;
     const int keepH = rs.sortHits;
+    // the shapes of the per-bounce kernels are timed: a trial short enough for
+    // the one kernel would tell nothing apart
+    struct TailOff {
+        bool& tail;
+        explicit TailOff(bool& t) : tail(t) { tail = false; }
+        ~TailOff() { tail = true; }
+    } tailOff(rs.tail);
     rs.quantNodes = 0;
     b.quantNodes = 0;
     rs.sortHits = 0;

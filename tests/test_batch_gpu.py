@@ -4,6 +4,7 @@ no launch shape changes any result."""
 import numpy as np
 import pytest
 
+from ratbite_amd import _lib as L
 from ratbite_amd import scenes
 from ratbite_amd.renderer import Renderer, render_batch
 
@@ -122,6 +123,26 @@ def test_autotune_keeps_results(ctx):
     r.render(spp=8, offset=0)
     assert np.array_equal(a, r.accum())
     r.set_tuning()
+
+
+def test_autotune_times_the_kernels_that_it_tunes():
+    # a trial of few paths would run in the one kernel that has none of the
+    # settings: while tuning every path goes through the per-bounce kernels
+    import ratbite_amd
+    with ratbite_amd.Context(0) as c:
+        r = Renderer(scenes.cornell(width=24, height=16, spp=1), ctx=c)
+        queued = np.zeros(8, np.uint32)
+
+        def read():
+            c.check(L.lib().rbh_test_queued(c.h, L.ptr(queued), len(queued)))
+            return queued[0]
+
+        r.render(spp=1, offset=0)
+        assert read() == 0
+        r.autotune(trial_spp=1)
+        assert read() == 24 * 16
+        r.render(spp=1, offset=0)
+        assert read() == 0
 
 
 def test_set_tuning_without_arguments_is_the_librarys_own():
