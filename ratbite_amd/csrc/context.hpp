@@ -189,7 +189,7 @@ struct rbh_context {
     rbh::RenderState rs;
     rbh_stats stats{};
     void* guide = nullptr;    // guiding state (guide.hip)
-    rbh::DevBuf guideRecords, guideOutputs;   // a caller's records on the device, and their outputs
+    rbh::DevBuf guideRecords, guideOutputs;   // a caller's records on the device, and their outputs (bounded: guide.hip)
     std::shared_ptr<rbh::CopyPool> copyPool;   // the device's threads for large host copies, from the first one on
     bool copyPoolFailed = false;
 };

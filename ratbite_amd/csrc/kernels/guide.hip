@@ -755,6 +755,17 @@ int rbh_guide_get_params(rbh_ctx c, float* params, uint32_t n) {
     return RBH_OK;
 }
 
+// The record and output buffers of a call stay on the context, up to this size
+// each (2M records in, 800k records' outputs); larger ones go with the call.
+constexpr size_t kKeptBytes = (size_t)128 << 20;
+struct KeptBuffers {
+    rbh_ctx c;
+    ~KeptBuffers() {
+        for (DevBuf* b : {&c->guideRecords, &c->guideOutputs})
+            if (b->bytes > kKeptBytes) b->release();
+    }
+};
+
 static int stage_records(rbh_ctx c, const float* recs, uint32_t n) {
     DevBuf& buf = c->guideRecords;
     RBH_ALLOC(c, buf, (size_t)std::max<uint32_t>(n, 1) * kRec * 4);
@@ -765,6 +776,7 @@ static int stage_records(rbh_ctx c, const float* recs, uint32_t n) {
 int rbh_guide_gradient(rbh_ctx c, const float* recs, uint32_t n, float* grad, float* loss) {
     if (!c || !recs || !grad || n == 0) return RBH_ERR_INVALID;
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
+    const KeptBuffers kept{c};
     DevBuf gbuf;
     int rc = stage_records(c, recs, n);
     if (rc) return rc;
@@ -780,6 +792,7 @@ int rbh_guide_gradient(rbh_ctx c, const float* recs, uint32_t n, float* grad, fl
 int rbh_guide_train(rbh_ctx c, const float* recs, uint32_t n, uint32_t batch, uint32_t steps, float* lastLoss) {
     if (!c || !recs || n == 0 || batch == 0) return RBH_ERR_INVALID;
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
+    const KeptBuffers kept{c};
     int rc = stage_records(c, recs, n);
     if (rc) return rc;
     float l = 0.0f;
@@ -869,6 +882,7 @@ static int infer(rbh_ctx c, const float* recs, uint32_t n, float* out, bool fp8)
     if (!gs(c).configured) return fail(c, RBH_ERR_STATE, "rbh_guide_configure first");
     if (n == 0) return RBH_OK;
     GuideState& g = gs(c);
+    const KeptBuffers kept{c};
     int rc = stage_records(c, recs, n);
     if (rc) return rc;
     DevBuf &d = c->guideRecords, &o = c->guideOutputs;

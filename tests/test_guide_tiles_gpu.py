@@ -2,6 +2,7 @@
 one workgroup per CU: gradient and loss against the FP64 oracle that rounds
 activations, weights and gradients to bfloat16 where the kernel stores them."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -31,3 +32,33 @@ def test_gradient_at_tile_edges(ctx, n):
     again = np.zeros_like(grad)
     ctx.check(L.lib().rbh_guide_gradient(ctx.h, L.ptr(rec), n, L.ptr(again), ctypes.byref(loss)))
     assert np.array_equal(grad, again)
+
+
+def test_large_calls_give_their_memory_back():
+    # a million records: 64 MB of input, 164 MB of output; buffers above 128 MiB
+    # go with the call
+    import ratbite_amd
+    rt = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n = 1000003
+    rec = np.tile(_records(1, np.random.default_rng(2)), (n, 1))
+    out = np.zeros((n, L.GUIDE_OUTPUTS), np.float32)
+    with ratbite_amd.Context(0) as c:
+        _configure(c)
+        # (large enough that the threads of the host copies have their queues)
+        c.call("rbh_guide_infer", L.ptr(rec), 50000, L.ptr(out))
+        one = out[0].copy()
+        free = free_bytes()
+        for call in ("rbh_guide_infer", "rbh_guide_infer_fp8", "rbh_guide_infer"):
+            c.call(call, L.ptr(rec), n, L.ptr(out))
+            # (the driver hands freed memory back a little later)
+            end = time.monotonic() + 10.0
+            while free - free_bytes() > 130 << 20 and time.monotonic() < end:
+                time.sleep(0.05)
+            assert free - free_bytes() <= 130 << 20, call
+        assert np.array_equal(out[0], one) and np.array_equal(out[-1], one)
