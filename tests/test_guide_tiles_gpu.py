@@ -20,14 +20,24 @@ def test_gradient_at_tile_edges(ctx, n):
     p = _params(5, scale_out=2.0)
     _set(ctx, p)
     rec = _records(n, np.random.default_rng(100 + n))
+    # the last record, alone in its tile for most of these sizes, weighs as
+    # much as all others together
+    rec[-1, 14] = max(float(rec[:-1, 14].sum()), 1.0)
     grad, loss = np.zeros(L.GUIDE_PARAMS, np.float32), ctypes.c_float()
     ctx.check(L.lib().rbh_guide_gradient(ctx.h, L.ptr(rec), n, L.ptr(grad), ctypes.byref(loss)))
     l_ref, g_ref = G.loss_grad(G.unflatten(p.astype(np.float64)), rec.astype(np.float64), emulate_bf16=True)
     ref = G.flatten(g_ref)
     # a value within FP32 rounding of the middle of two bfloat16 values may
     # round the other way: 2^-8 of single terms, and five layers of them
-    assert np.linalg.norm(grad - ref) / np.linalg.norm(ref) < 5 * 2.0 ** -8
+    bound = 5 * 2.0 ** -8
+    assert np.linalg.norm(grad - ref) / np.linalg.norm(ref) < bound
     assert abs(loss.value - l_ref) <= 2e-3 * abs(l_ref) + 1e-5
+    if n > 1:
+        # the bounds tell the last record from a missing or a repeated one
+        for wrong in (rec[:-1], np.concatenate([rec[:-1], rec[-2:-1]])):
+            l_wrong, g_wrong = G.loss_grad(G.unflatten(p.astype(np.float64)), wrong.astype(np.float64), emulate_bf16=True)
+            assert np.linalg.norm(G.flatten(g_wrong) - ref) / np.linalg.norm(ref) > 4 * bound
+            assert abs(l_wrong - l_ref) > 2 * (2e-3 * abs(l_ref) + 1e-5)
     # partial sums in a fixed order: the same call gives the same bits
     again = np.zeros_like(grad)
     ctx.check(L.lib().rbh_guide_gradient(ctx.h, L.ptr(rec), n, L.ptr(again), ctypes.byref(loss)))
