@@ -70,25 +70,34 @@ def test_collect_train_and_gain(ctx):
 
     e_plain = err(no_drop=True)
     e_untr = err(guided=True)
-    losses = []
-    for it in range(32):
-        r.render(spp=8, offset=100000 + 8 * it, guided=True, collect=True)
-        if it == 0:
-            recs = r.guide_records()
-            assert len(recs) > 1000
-            assert np.all(np.isfinite(recs)) and np.all(recs[:, 14] >= 0)
-            d = recs[:, 11:14]
-            assert np.allclose(np.linalg.norm(d, axis=1), 1.0, atol=1e-4)
-            assert np.all((recs[:, 0:3] >= 0) & (recs[:, 0:3] <= 1))
-        losses.append(r.train_guide(batch=1 << 16, steps=20))
-    e_tr = err(guided=True)
-    print("losses", np.round(losses, 3), flush=True)
+    trained, curves = [], []
+    for training in range(5):
+        r.configure_guide(seed=5, lr=2e-3, capacity=1 << 21)
+        losses = []
+        for it in range(32):
+            r.render(spp=8, offset=100000 + 8 * it, guided=True, collect=True)
+            if it == 0:
+                recs = r.guide_records()
+                assert len(recs) > 1000
+                assert np.all(np.isfinite(recs)) and np.all(recs[:, 14] >= 0)
+                d = recs[:, 11:14]
+                assert np.allclose(np.linalg.norm(d, axis=1), 1.0, atol=1e-4)
+                assert np.all((recs[:, 0:3] >= 0) & (recs[:, 0:3] <= 1))
+            losses.append(r.train_guide(batch=1 << 16, steps=20))
+        curves.append(losses)
+        trained.append(err(guided=True))
+        print("losses", np.round(losses, 3), flush=True)
+    e_tr = np.median(trained, axis=0)
     print("relMSE at 128 spp (mean of 6 renders, raw / 0.1%%-trimmed) vs 32768-spp plain: plain %.4g / %.4g, "
-          "guided untrained %.4g / %.4g, guided trained %.4g / %.4g" % (*e_plain, *e_untr, *e_tr), flush=True)
-    assert np.mean(losses[-8:]) < np.mean(losses[:4])
+          "guided untrained %.4g / %.4g, guided trained (median of 5) %.4g / %.4g" % (*e_plain, *e_untr, *e_tr), flush=True)
+    curves = np.array(curves)
+    assert np.mean(curves[:, -8:]) < np.mean(curves[:, :4])
     assert e_tr[1] < e_untr[1]
-    # the trained guide beats BSDF sampling at equal samples (0.098 vs 0.125
-    # measured); the margin is several times the spread of six renders
+    # the trained guide beats BSDF sampling at equal samples. The records of a
+    # collecting render are in no fixed order, so trainings from one seed
+    # differ: of 200, the trimmed ratio to plain has the median 0.765 and 7%
+    # are above 0.9 (the largest 1.12); the median of five is above 0.9 in
+    # 0.3% (10 x 0.07^3)
     assert e_tr[1] < 0.9 * e_plain[1]
 
 
