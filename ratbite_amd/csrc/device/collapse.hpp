@@ -48,13 +48,9 @@ __device__ __forceinline__ float half_area(const Box& b) {
 // position on the axis (all vertices NaN) is open to that side.
 template <bool UPPER>
 __device__ __forceinline__ uint16_t grid_plane(float p, float o, int e) {
-    const float outside = UPPER ? INFINITY : -INFINITY;
-    float q = p == p ? p : outside;
-    if (fabsf(p) < INFINITY) {
-        const double x = ldexp((double)p - (double)o, -e);
-        q = (float)(UPPER ? ceil(x) : floor(x));
-    }
-    return __builtin_bit_cast(uint16_t, (_Float16)q);
+    const double x = ldexp((double)p - (double)o, -e);
+    const float q = (float)(UPPER ? ceil(x) : floor(x));
+    return __builtin_bit_cast(uint16_t, (_Float16)(q == q ? q : UPPER ? INFINITY : -INFINITY));
 }
 
 // The 11-bit form of a four-wide node whose inner children come first. Grid
