@@ -57,7 +57,7 @@ struct GuideState {
     void* bias = nullptr;              // float[kBiasPad]
     void* partials = nullptr;          // float[blocks][kParams]
     size_t partialBlocks = 0;
-    void* scalars = nullptr;           // floats: loss and weight sums, then their partial sums per block
+    void* scalars = nullptr;           // floats: the loss, the weight sum of a collected set, then the partial sums of weights and losses per block
     void* records = nullptr;           // pending records of a collecting render (float[cap][24])
     void* trainRecs = nullptr;         // finished training records (float[cap][kRec])
     void* recCount = nullptr;          // uint32 counter

@@ -200,7 +200,8 @@ __device__ __forceinline__ void store_grads(float* __restrict__ part, int l, int
     }
 }
 
-constexpr int kScalars = 4;         // floats ahead of the partial sums: weight sum, loss, collected weight sum
+// floats ahead of the partial sums in GuideState::scalars
+enum : int { GS_LOSS = 0, GS_COLLECTED = 1, kScalars = 4 };   // the loss; the weight sum of a collected set
 constexpr int kSumBlocks = 256;     // partial weight sums, then as many partial losses
 
 __global__ __launch_bounds__(kTrainBlock) void k_guide_train(const float* __restrict__ recs, uint32_t n,
@@ -662,13 +663,13 @@ int run_train(rbh_ctx c, const float* drecs, uint32_t n, int mode, float* gradOu
     hipLaunchKernelGGL(k_guide_reduce, dim3((kParams + kReduceParams - 1) / kReduceParams), dim3(256), 0, c->stream,
                        dptr<float>(g.partials), blocks, mode, dptr<float>(g.master), dptr<float>(g.adamM),
                        dptr<float>(g.adamV), g.lr, g.beta1, g.beta2, g.eps, bc1, bc2, dptr<bf16>(g.wf), dptr<bf16>(g.wt),
-                       dptr<float>(g.bias), gradOut, lpart, sc + 1);
+                       dptr<float>(g.bias), gradOut, lpart, sc + GS_LOSS);
     RBH_HIP(c, hipGetLastError());
     if (lossOut) {
-        float tmp[4];
-        RBH_HIP(c, hipMemcpyAsync(tmp, sc, 16, hipMemcpyDeviceToHost, c->stream));
+        float l = 0.0f;
+        RBH_HIP(c, hipMemcpyAsync(&l, sc + GS_LOSS, sizeof(l), hipMemcpyDeviceToHost, c->stream));
         RBH_HIP(c, hipStreamSynchronize(c->stream));
-        *lossOut = tmp[1];
+        *lossOut = l;
     }
     return RBH_OK;
 }
@@ -849,7 +850,7 @@ static int prepare_collected(rbh_ctx c, uint32_t n, uint32_t* m) {
     float* out = static_cast<float*>(g.records);
     const int blocks = (int)std::min<uint32_t>(4096u, (k + 255u) / 256u);
     hipLaunchKernelGGL(k_gather_records, dim3(blocks), dim3(256), 0, c->stream, recs, idx.as<uint32_t>(), k, stride, out);
-    float* sum = dptr<float>(g.scalars) + 2;
+    float* sum = dptr<float>(g.scalars) + GS_COLLECTED;
     for (int pass = 0; pass < 2; ++pass) {
         hipLaunchKernelGGL(k_zero_f32, dim3(1), dim3(64), 0, c->stream, sum, 1);
         hipLaunchKernelGGL(k_weight_sum, dim3(256), dim3(256), 0, c->stream, out, k, sum);

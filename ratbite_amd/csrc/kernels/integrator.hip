@@ -486,7 +486,7 @@ __global__ __launch_bounds__(kShadeBlock, WAVES) void k_shade(Frame1 f, uint32_t
 // 1080p x 64 spp of 4.1M triangles 114.3 / 114.1 / 116.3 / 122.3 ms.
 constexpr uint32_t kTailPaths = 65536u;
 // Waves per SIMD: a tail is up to 4096 waves, two rounds at two waves per SIMD
-// (227 registers) and better off with a few spills and three: feature scene
+// (231 registers) and better off with a few spills and three: feature scene
 // 333x187x8 2.27 -> 2.17 ms, edit of 1M triangles with a 640x360 preview 2.85 ->
 // 2.62 ms (four waves: 2.24 / 2.85 ms). Up to kFewPaths are resident at once
 // either way, and the registers shorten their chain: 64x64 preview 0.485 against

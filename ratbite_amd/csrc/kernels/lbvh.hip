@@ -12,15 +12,16 @@
 //   5. boxes bottom up: a workgroup takes 2048 consecutive leaves, writes their
 //      triangle records and climbs the hierarchy in LDS (of a node's two
 //      children the second to arrive merges them) as far as the nodes' leaf
-//      ranges stay within the workgroup's; one workgroup then climbs the few
-//      nodes above (no cross-XCD fences: only kernel boundaries order the
-//      two). A node is emitted where its children meet, as the 64-byte
+//      ranges stay within the workgroup's; above them a workgroup climbs for
+//      every group of 32 such tiles, and one for the few nodes above the
+//      groups (no cross-XCD fences: only kernel boundaries order the three). A node is emitted where its children meet, as the 64-byte
 //      two-child node with both child boxes
 //   6. collapse into 128-byte four-wide nodes (with full boxes and on an
 //      11-bit grid), top down: a four-wide node
 //      takes its binary node's children and keeps opening the inner child
-//      with the largest box surface until it has four. The same workgroup
-//      runs the upper levels, then one wave per subtree finishes. The inner
+//      with the largest box surface until it has four (device/collapse.hpp).
+//      The same workgroup runs the upper levels, then waves take the subtrees
+//      below, in rounds that spread what is left over all of them again. The inner
 //      children of a four-wide node have consecutive indices in slot order,
 //      from a range of indices that belongs to the node alone
 // Every root-to-leaf path strictly lengthens the common key prefix, so the

@@ -109,9 +109,9 @@ def test_four_wide_tree_matches_binary(ctx):
 
 @pytest.mark.parametrize("which", ["soup", "spheres"])
 def test_quantised_nodes_match_full_precision(ctx, which):
-    # the 64-byte nodes hold conservative 8-bit child boxes: they prune less
-    # but never a triangle the ray hits before its current best, so the
-    # closest t is bit-identical and the any-hit occlusion the same
+    # the grid nodes hold conservative child boxes: they prune less but never
+    # a triangle the ray hits before its current best, so the closest t is
+    # bit-identical and the any-hit occlusion the same
     rng = np.random.default_rng(31)
     if which == "soup":
         c = rng.uniform(-5, 5, (3000, 3))
